@@ -1044,7 +1044,7 @@ __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, con
             const int r = pos[k];
             const bool below = r > lo0[k];  // then beam[r-1] and cand[d-r] both exist
             const float a = bk[2 * (below ? r : 1) - 2], b = mk[2 * (below ? dd[k] - r : 0)];
-            tie |= below && a == b && a != FLT_MAX;
+            tie |= below & (a == b) & (a != FLT_MAX);
             rr[k] = r;
         }
         replay = any_lane(tie);
@@ -1118,17 +1118,18 @@ __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, con
         for (int s2 = 0; s2 < 4; ++s2) {
             ina[s2] = s2 < na;
             slot[k][s2] = ina[s2] ? bp[tb + s2] : ms[cb + s2 - na];
-            pos[k][s2] = dl[k];
+            pos[k][s2] = dl[k] + s2;
         }
+        // a candidate slot u that goes before a beam slot s2 < u swaps their
+        // order (masks and carries, no branch)
 #pragma unroll
         for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
             for (int u = s2 + 1; u < 4; ++u) {
                 // slots at or past nsl are unused: they never count
-                const bool cross = ina[s2] && !ina[u];
-                const bool first = !cross || !(pair_key(slot[k][u]) < pair_key(slot[k][s2]));
-                pos[k][u] += first ? 1 : 0;
-                pos[k][s2] += (!first && u < nsl[k]) ? 1 : 0;
+                const bool ahead = ina[s2] & !ina[u] & (pair_key(slot[k][u]) < pair_key(slot[k][s2]));
+                pos[k][u] -= ahead ? 1 : 0;
+                pos[k][s2] += (ahead & (u < nsl[k])) ? 1 : 0;
             }
     }
     // every lane has read its inputs before any output overwrites them
@@ -1235,9 +1236,10 @@ __device__ __forceinline__ uint32_t hash_next(uint32_t b, uint32_t nb) { return 
 
 // (min of the four XORs is zero iff one slot equals the key: integer ops the
 // compiler keeps as such, where four compares became packed 16-bit flags)
-__device__ __forceinline__ bool bucket_has(uint4 s, uint32_t key) {
-    return min(min(s.x ^ key, s.y ^ key), min(s.z ^ key, s.w ^ key)) == 0u;
+__device__ __forceinline__ uint32_t bucket_diff(uint4 s, uint32_t key) {
+    return min(min(s.x ^ key, s.y ^ key), min(s.z ^ key, s.w ^ key));
 }
+__device__ __forceinline__ bool bucket_has(uint4 s, uint32_t key) { return bucket_diff(s, key) == 0u; }
 
 __device__ __forceinline__ bool bucket_open(uint4 s) { return static_cast<int32_t>(s.w) < 0; }
 
@@ -1251,12 +1253,14 @@ __device__ __forceinline__ uint32_t hash_insert(uint32_t *t, uint32_t nb, uint32
     const uint4 *t4 = reinterpret_cast<const uint4 *>(t);
     const uint32_t ba = hash_home(key, nb), bb = hash_alt(key, nb);
     // a failed CAS means another lane filled a slot of one of the two
-    // buckets: at most 8 passes before both are full
+    // buckets: at most 8 passes before both are full.  Both buckets are read
+    // together and compared at once (two LDS round trips a pass).
+#pragma unroll 1
     for (int pass = 0; pass < 9; ++pass) {
         const uint4 sa = t4[ba], sb = t4[bb];
-        if (bucket_has(sa, key) || bucket_has(sb, key)) return 0;
+        if (min(bucket_diff(sa, key), bucket_diff(sb, key)) == 0u) return 0;
         const uint32_t fa = bucket_free(sa), fb = bucket_free(sb);
-        if (fa == 0u && fb == 0u) break;
+        if ((fa | fb) == 0u) break;
         const bool alt = fb > fa;
         const uint32_t slot = 4u * (alt ? bb : ba) + 4u - (alt ? fb : fa);
         const uint32_t old = atomicCAS(&t[slot], kMaxIndex, key);
@@ -1650,12 +1654,19 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
     bool anyp = false;
 #pragma unroll
     for (int s = 0; s < NK; ++s) {
-        // branch-free: every lane reads both buckets (indices always in range)
+        // branch-free: every lane reads both buckets (indices always in
+        // range), and one minimum over the eight XORs decides.  Bound by the
+        // latency of the reads: written as "in one bucket or the other" it
+        // compiled to a branch per key with the second read behind it, eight
+        // dependent LDS round trips for four keys instead of one.  With the
+        // same change in hash_insert and merge_path: 2,000 queries at d 128,
+        // beam 1024 2.02 -> 1.92 ms, 777 at d 200 0.646 -> 0.602 ms, 10,000
+        // at d 96, degree 16, beam 512 2.56 -> 2.46 ms
         b[s] = hash_alt(key[s], nb);
         const uint4 sa = t4[hash_home(key[s], nb)], sb = t4[b[s]];
-        const bool has = bucket_has(sa, key[s]) || bucket_has(sb, key[s]);
-        pend[s] = test[s] && !has && both_full(sa, sb);
-        test[s] = test[s] && !has;  // contained: not a fresh child
+        const bool fresh = min(bucket_diff(sa, key[s]), bucket_diff(sb, key[s])) != 0u;
+        test[s] = test[s] & fresh;  // contained: not a fresh child
+        pend[s] = test[s] & both_full(sa, sb);
         anyp |= pend[s];
     }
     if (!any_lane(anyp)) return;
