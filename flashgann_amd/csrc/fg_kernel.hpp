@@ -38,9 +38,13 @@ constexpr int kMaxPaddedDim = 2048;
 constexpr float kPhase1Rho = 0.25f;   // PHASE1_RHO
 constexpr float kRhoMax = 0.99f;      // RHO_MAX
 constexpr int kStallIters = 4;        // TOP1_WARMUP_STALL_ITERS
-constexpr int kPlanes = 6;            // q in [1, 64]: q - 1 needs 6 bit-planes
-constexpr int kWrapPlane = 6;         // chunks whose four levels are all 64
-constexpr int kZeroPlane = 7;         // levels that are 0 (a degenerate query only)
+
+// The prepared query in LDS, for W = padded_dim / 32 code words: three digit
+// rows of 16 bytes per word (prepare_query), a row of zeros, then the W wrap
+// words (the chunks whose four levels are all 64).
+__host__ __device__ constexpr uint32_t prep_zero_off(uint32_t W) { return 48u * W; }
+__host__ __device__ constexpr uint32_t prep_wrap_off(uint32_t W) { return 48u * W + 16u; }
+__host__ __device__ constexpr uint32_t prep_words(uint32_t W) { return 13u * W + 4u; }
 
 // ------------------------------------------------------------ host+device
 
@@ -106,17 +110,15 @@ __host__ __device__ inline int keep_count_for_expander(uint32_t active, int thet
 // one reset interval of inserts, <= 32 per 8-task round, + the entry point).
 // A table with more slots than that never fills, so it answers every
 // membership query exactly like the reference's 2^11-entry table
-// (utils.cuh:137-151), which never fills either.  The smallest table keeps
-// that worst case at <= 99% load with at least one slot to spare (an insert
-// always finds a free slot, a lookup's walk always meets one); the roomiest
-// at <= 90% (fewer lookups that walk on).  visited_buckets() picks between
-// them.
+// (utils.cuh:137-151), which never fills either.  The smallest table has one
+// slot more than that worst case (an insert always finds a free slot, a
+// lookup's walk always meets one); the roomiest holds it at <= 90% load (fewer
+// lookups that walk on).  visited_buckets() picks between them.
 __host__ __device__ inline uint32_t visited_keys_max(uint32_t beam, uint32_t degree) {
     return beam + 16u * 32u * ((degree + 31) / 32) + 1u;
 }
 __host__ __device__ inline uint32_t visited_buckets_min(uint32_t beam, uint32_t degree) {
-    const uint32_t slots = (visited_keys_max(beam, degree) * 100u + 98u) / 99u + 1u;
-    return (slots + 3u) / 4u;
+    return (visited_keys_max(beam, degree) + 1u + 3u) / 4u;
 }
 __host__ __device__ inline uint32_t visited_buckets_roomy(uint32_t beam, uint32_t degree) {
     const uint32_t slots = (visited_keys_max(beam, degree) * 10u + 8u) / 9u;
@@ -124,7 +126,7 @@ __host__ __device__ inline uint32_t visited_buckets_roomy(uint32_t beam, uint32_
 }
 
 struct LdsLayout {
-    uint32_t hash_off, beam_off, msort_off, plane_off, scratch_off, prof_off, total, total_prof, team_off,
+    uint32_t hash_off, beam_off, msort_off, prep_off, scratch_off, prof_off, total, total_prof, team_off,
         total_team;
 };
 
@@ -134,7 +136,7 @@ struct LdsLayout {
 // up).  The stages fill slots 0..31 in any order; the merge reads them into
 // registers, sorts them and writes them back sorted before it merges.
 constexpr int kMsortHi = 35;
-constexpr uint32_t kMsortPairs = 38;
+constexpr uint32_t kMsortPairs = 37;
 // Beam: (distance, id) pairs at indices -1 .. pbeam + kBeamPad - 1: a
 // -FLT_MAX sentinel, the pbeam entries, a FLT_MAX sentinel at pbeam, then pad
 // entries (segment reads may run up to 3 past pbeam; the merge's unused
@@ -150,7 +152,7 @@ struct TeamBlock {
     // number of expanders; then the exact batch's size and list kind
     uint32_t stop, theta, nexp, kth_bits, rho_bits, ex_n, ex_alist, pad0;
     // per query (written once): the quantised query's constants
-    uint32_t sum_q, qwidth_bits, qlow_bits, any_wrap, any_zero;
+    uint32_t sum_q, qwidth_bits, qlow_bits, any_wrap, pad2;
     // the helper's work counters (counting build)
     uint32_t c_ids, c_est, pad1;
     // the helper's stage-II results: kept-lane masks and child ids of its
@@ -173,33 +175,33 @@ __device__ __forceinline__ void team_stop(TeamBlock *tb, int lane) {
 
 
 // Per-query LDS: visited table and beam (aliased by the rotated query during
-// preparation), the candidate pairs, 8 x B/32 plane words and a small
+// preparation), the candidate pairs, the prepared query and a small
 // scratch area (32-entry child list + parent ids and distances).  The raw
 // query is read from global memory, where it stays cached (the fixed
 // geometries keep it in registers through the loop).
 __host__ __device__ constexpr LdsLayout lds_layout(uint32_t dim, uint32_t padded_dim, uint32_t pbeam,
                                                    uint32_t buckets) {
     // fixed-size regions first (compile-time offsets for a fixed geometry),
-    // then the beam-dependent visited table and beam
+    // then the beam-dependent ones: the beam, then the visited table at the
+    // next multiple of 16 (this order wastes no padding: at d 128, beam 512
+    // the total is 7 granules to the byte)
     LdsLayout L{};
     uint32_t off = 0;
-    L.msort_off = off;
-    off += kMsortPairs * 8u;
     (void)dim;
-    L.plane_off = off;
-    off += 8u * (padded_dim / 32u) * 4u;
+    L.prep_off = off;
+    off += prep_words(padded_dim / 32u) * 4u;
     L.scratch_off = off;
     off += (32u + 2u * 8u) * 4u;
-    off = (off + 15u) & ~15u;
-    L.hash_off = off;
+    L.msort_off = off;
+    off += kMsortPairs * 8u;
     // during query preparation the rotated query (padded_dim floats) spans the
-    // visited table and the beam, which are initialised after it
-    uint32_t hash_bytes = buckets * 16u;
-    const uint32_t beam_bytes = (pbeam + 1u + kBeamPad) * 8u;
-    if (hash_bytes + beam_bytes < padded_dim * 4u) hash_bytes = (padded_dim * 4u - beam_bytes + 15u) & ~15u;
-    off += hash_bytes;
+    // beam and the visited table, which are initialised after it
     L.beam_off = off;
     off += (pbeam + 1u + kBeamPad) * 8u;
+    off = (off + 15u) & ~15u;
+    L.hash_off = off;
+    off += buckets * 16u;
+    if (off < L.beam_off + padded_dim * 4u) off = L.beam_off + padded_dim * 4u;
     L.total = (off + 15u) & ~15u;
     // phase timers of the profiling build only, past the end of the rest
     L.prof_off = L.total;
@@ -270,8 +272,8 @@ struct SearchParams {
 // words), the work counters (6), the candidate span, the split flag and the
 // pick's start (beams over 256), then the pbeam beam pairs and the 32
 // candidate pairs, then the prepared query: low, width, sum_q, a pad word and
-// the 8 planes of W = padded_dim / 32 words (so the second slice does not
-// rotate and quantise the query again, nor read the entry point's row).
+// its LDS block (prep_words: the second slice does not rotate and quantise
+// the query again, nor read the entry point's row).
 // slice_keys holds the key (bits of a finite float: the best distance so far)
 // of each suspended query and kSliceDone (a NaN pattern, never a key) for a
 // query the first slice finished.
@@ -279,7 +281,7 @@ constexpr uint32_t kSliceHeader = 64;
 constexpr uint32_t kSliceFixed = 20;  // 2 + 9 + 6 + 2 + 1 (the pick's start, beams over 256)
 __host__ __device__ inline uint32_t slice_prep_offset(uint32_t pbeam) { return kSliceFixed + 2u * (pbeam + 32u); }
 __host__ __device__ inline uint32_t slice_words(uint32_t pbeam, uint32_t padded_dim) {
-    return slice_prep_offset(pbeam) + 4u + 8u * (padded_dim / 32u);
+    return slice_prep_offset(pbeam) + 4u + prep_words(padded_dim / 32u);
 }
 constexpr uint32_t kSliceDone = 0xFFFFFFFFu;
 constexpr int kSliceMaxQueries = 16384;  // the one-workgroup order kernel holds every query's bin in LDS
@@ -545,13 +547,20 @@ __device__ __forceinline__ void lead_sync() {
 
 // utils.cuh:790-939 for one wave: rotate (x*signs, pad, FWHT len = 1..B/2 with
 // butterflies (u+v, u-v)), min/max, width = (hi-lo)*fl(1/63), q = round(fma(
-// y-lo, 1/width, 0.5)) (NaN -> 0), then the 6 popcount planes of q - 1, the
-// level-0 mask and the chunks whose uint8 LUT entry would wrap.  Writes
-// planes (8 x W words) and returns low, width, sum_q.  `rot` is LDS scratch
-// of B floats.
+// y-lo, 1/width, 0.5)) (NaN -> 0), then the prepared query's LDS block: the
+// levels as digit rows for the matrix unit and the chunks whose uint8 LUT entry
+// would wrap.  Returns low, width, sum_q.  `rot` is LDS scratch of B floats.
+//
+// Digit rows.  A code bit contributes its dimension's level q in [0, 64], and
+// q = d0 + 5 d1 + 25 d2 with digits -2 .. 2 (d2 up to 3).  Row t of code word
+// w holds digit t of the word's 32 dimensions as 4-bit floats (E2M1), in the
+// order in which raw_mfma spreads a code word's bits: dword r, nibble i is
+// bit 4 i + r of the word.  There a set bit stands as the 4-bit float 0.5, 1,
+// 2 and 0.5 for r = 0 .. 3, so the digits are stored times 2, 1, 1/2 and 2:
+// every product is the digit itself.
 template <int NW = 1>
 __device__ __forceinline__ void prepare_query(const float *__restrict__ query, const float *__restrict__ signs, int dim,
-                              int B, float *rot, float *qv, uint32_t *planes, float &low_out,
+                              int B, float *rot, float *qv, uint32_t *prep, float &low_out,
                               float &high_out, float &width_out, int &sumq_out, uint8_t *qdump) {
     const int lane = lane_id();
     for (int i = lane; i < B; i += 64) {
@@ -595,23 +604,32 @@ __device__ __forceinline__ void prepare_query(const float *__restrict__ query, c
         const uint32_t q = isnan(scaled) ? 0u : static_cast<uint32_t>(roundf(scaled));
         if (qdump) qdump[i] = static_cast<uint8_t>(q);
         sum += static_cast<int>(q);
-        // planes of q - 1: a code's sum over its set bits is then
-        // popcount(code) + sum_p 2^p popcount(code & plane_p), minus the set
-        // bits at level 0 (plane kZeroPlane; only a query whose rotation is
-        // constant or not finite has such levels, and then all of them)
-        const uint32_t r = q != 0u ? q - 1u : 0u;
-        for (int p = 0; p < kPlanes; ++p) {
-            const uint64_t m = ballot(((r >> p) & 1u) != 0u);
-            if (nl == 0) planes[p * W + w] = half_bits(m, h);
+        // this lane's dimension sits at bit nl of word w: dword nl & 3, nibble
+        // nl >> 2.  The 4-bit floats of 0 .. 3 times 2, 1, 1/2, as nibbles:
+        const uint32_t r = static_cast<uint32_t>(nl) & 3u;
+        const uint32_t table = r == 1u ? 0x5420u : r == 2u ? 0x3210u : 0x7640u;
+        // (a spread too small for fp32, whose inverse overflows, gives levels
+        // past 64, which the width of such a query makes immaterial)
+        int rest = static_cast<int>(min(q, 64u));
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int up = (rest + 2) / 5, digit = t < 2 ? rest - 5 * up : rest;
+            rest = up;
+            const uint32_t mag = static_cast<uint32_t>(digit < 0 ? -digit : digit);
+            const uint32_t code = ((table >> (4u * mag)) & 15u) | (digit < 0 ? 8u : 0u);
+            uint32_t d = code << (4u * (static_cast<uint32_t>(nl) >> 2));
+            d |= xshfl(d, 4);
+            d |= xshfl(d, 8);
+            d |= xshfl(d, 16);
+            if (nl < 4) prep[(3 * w + t) * 4 + nl] = d;
         }
-        const uint64_t zm = ballot(q == 0u);
-        if (nl == 0) planes[kZeroPlane * W + w] = half_bits(zm, h);
         // a chunk's full-nibble LUT entry is (q0+q1+q2+q3) mod 256 (utils.cuh:913-917)
         uint32_t s = q + xshfl(q, 1);
         s += xshfl(s, 2);
         const uint64_t wm = ballot(s >= 256u);
-        if (nl == 0) planes[kWrapPlane * W + w] = half_bits(wm, h);
+        if (nl == 0) prep[prep_wrap_off(W) / 4u + w] = half_bits(wm, h);
     }
+    if (lane < 4) prep[prep_zero_off(W) / 4u + lane] = 0u;
     sumq_out = uni(wave_sum(sum));
     low_out = lo;
     high_out = hi;
@@ -619,131 +637,196 @@ __device__ __forceinline__ void prepare_query(const float *__restrict__ query, c
     lead_sync<NW>();
 }
 
-// popcount(x) + acc as one v_bcnt_u32_b32.  Written as an instruction so a
-// chain of them stays a chain: as plain additions the compiler splits it into
-// popcounts from zero joined by three-input adds, two more instructions per
-// plane and code block.
-__device__ __forceinline__ uint32_t bcnt_acc(uint32_t x, uint32_t acc) {
-    uint32_t r;
-    asm("v_bcnt_u32_b32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(acc));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// Where a lane reads its part of the matrix operand that holds the prepared
+// query (raw_mfma): the address of code word 0's row, and the step from word
+// to word.
+struct LevelRows {
+    uint32_t at, step;
+};
+__device__ __forceinline__ LevelRows level_rows(uint32_t W) {
+    // operand row m = lane & 15 and K block g = lane >> 4: row 4 g + t of block
+    // g is digit row t (t < 3), every other row of the block zero
+    const uint32_t lane = static_cast<uint32_t>(lane_id());
+    const uint64_t diag = 0x7ull | 0x7ull << 20 | 0x7ull << 40 | 0x7ull << 60;
+    LevelRows r;
+    r.at = lane_in(diag) ? 16u * (lane & 3u) : prep_zero_off(W);
+    r.step = lane_in(diag) ? 48u : 0u;
     return r;
 }
 
-// raw = sum_cb LUT[cb][nibble] (utils.cuh:976-980) over code words [w0, w1):
-// popcount(code) + sum_p 2^p popcount(code & plane_p) (the planes hold
-// q - 1), less the set bits at level 0 and 256 per wrapped chunk.
-__device__ __forceinline__ int32_t raw_partial(const uint32_t *__restrict__ code, int w0, int w1,
-                                               const uint32_t *planes, int W) {
-    uint32_t acc[kPlanes];
+// raw = sum_cb LUT[cb][nibble] (utils.cuh:976-980) on the matrix unit, for
+// code words [w0, w0 + NWD) of NB neighbour codes per lane, added to acc: the
+// sum over a code's set bits of their dimensions' levels.
+//
+// One 16x16x128 product per code word and 64 lanes.  Each lane feeds its own
+// code: the word's 32 bits, spread over four dwords as 4-bit floats (three
+// ANDs, a shift and an AND), are column lane & 15 of K block lane >> 4, so a
+// column of the second operand holds the words of four lanes, one per block.
+// The first operand is block diagonal: row 4 g + t holds digit row t of the
+// query in block g only.  Result row 4 g + t of a column is then digit sum t
+// of the lane (g, column), and it lands in that lane's result register t:
+// no data crosses lanes.  All sums are of small whole numbers, exact in
+// fp32, so the order of the unit's additions does not matter.
+// A quarter of the operand is useful, but 5 vector instructions and one
+// matrix instruction replace 13 vector instructions (six bit-planes' AND and
+// popcount, and the code's own popcount) per word, and the search is bound by
+// vector issue where it fills the device and by its instruction chain where
+// it does not.  Measured with the scalar keep decisions that follow the
+// estimates (against popcounts and vector ones): d 128 beam 256, 10,000
+// queries 1.334 -> 1.281 ms, beam 1024, 2,000 queries 1.92 -> 1.87; d 960,
+// 1,000 queries 1.061 -> 0.997; d 1536, 10,000 queries 17.14 -> 16.68; d 100
+// degree 24 0.517 -> 0.456.
+template <int NB, int NWD>
+__device__ __forceinline__ void raw_mfma(const uint32_t (&c)[NB][NWD], const unsigned char *prep, LevelRows lr, int w0,
+                                         v4f (&acc)[NB]) {
+    // The query's rows are read GA words ahead of the products that take them
+    // (the barriers keep the compiler from sinking a read to its product, an
+    // LDS round trip a word).
+    constexpr int GA = NWD <= 4 ? NWD : (NB == 1 ? 4 : 2);
+    const unsigned char *at = prep + lr.at + static_cast<uint32_t>(w0) * lr.step;
+    int4 cur[GA], nxt[GA];
 #pragma unroll
-    for (int p = 0; p < kPlanes; ++p) acc[p] = 0;
-    uint32_t ones = 0, zeros = 0, wraps = 0;
-    for (int w = w0; w < w1; ++w) {
-        const uint32_t c = code[w];
-#pragma unroll
-        for (int p = 0; p < kPlanes; ++p) acc[p] += __popc(c & planes[p * W + w]);
-        ones += __popc(c);
-        zeros += __popc(c & planes[kZeroPlane * W + w]);
-        const uint32_t x = c & planes[kWrapPlane * W + w];
-        wraps += __popc(x & (x >> 1) & (x >> 2) & (x >> 3) & 0x11111111u);
+    for (int i = 0; i < GA; ++i) {
+        cur[i] = *reinterpret_cast<const int4 *>(at);
+        at += lr.step;
     }
-    uint32_t raw = ones - zeros;
 #pragma unroll
-    for (int p = 0; p < kPlanes; ++p) raw += acc[p] << p;
-    return static_cast<int32_t>(raw - 256u * wraps);
+    for (int w = 0; w < NWD; w += GA) {
+        if (w + GA < NWD) {
+#pragma unroll
+            for (int i = 0; i < GA; ++i) {
+                nxt[i] = *reinterpret_cast<const int4 *>(at);
+                at += lr.step;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < GA; ++i) {
+            const v8i a = {cur[i].x, cur[i].y, cur[i].z, cur[i].w, 0, 0, 0, 0};
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const uint32_t x = c[b][w + i];
+                const v8i k = {static_cast<int>(x & 0x11111111u), static_cast<int>(x & 0x22222222u),
+                               static_cast<int>(x & 0x44444444u), static_cast<int>((x >> 3) & 0x11111111u), 0, 0, 0, 0};
+                acc[b] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, k, acc[b], 4, 4, 0, 0, 0, 0);
+            }
+        }
+        if (w + GA < NWD) {
+#pragma unroll
+            for (int i = 0; i < GA; ++i) cur[i] = nxt[i];
+        }
+    }
 }
 
-// popcount(c) + sum_p 2^p popcount(c & plane_p) - popcount(c & zero plane)
-// over NB code words starting at word w0 (added to raw), and the count of
-// wrapped chunks among them (added to wraps).  NB is a compile-time width,
-// so the plane reads carry no per-step condition and can be issued ahead of
-// the popcounts that consume them.
-template <int NB>
-__device__ __forceinline__ void raw_span(const uint32_t *__restrict__ code, const uint32_t *planes, int W, int w0,
-                                         bool vec_ok, bool any_wrap, bool any_zero, uint32_t &raw, uint32_t &wraps) {
-    uint32_t c[NB];
-    if (vec_ok) {
+// d0 + 5 d1 + 25 d2
+__device__ __forceinline__ float raw_value(v4f a) { return fmaf(25.0f, a[2], fmaf(5.0f, a[1], a[0])); }
+
+// Whether any chunk of the prepared query wraps the reference's uint8 LUT entry
+// (utils.cuh:913-917; uniform).
+__device__ __forceinline__ uint32_t wraps_anywhere(const unsigned char *prep, int W) {
+    uint32_t any = 0u;
+    for (int w = lane_id(); w < W; w += 64) any |= reinterpret_cast<const uint32_t *>(prep + prep_wrap_off(W))[w];
+    return any_lane(any != 0u) ? 1u : 0u;
+}
+
+// Wrapped chunks whose four bits are set, among NWD words of one code.
+template <int NWD>
+__device__ __forceinline__ uint32_t wrap_count(const uint32_t (&c)[NWD], const unsigned char *prep, uint32_t W, int w0) {
+    const uint32_t *wp = reinterpret_cast<const uint32_t *>(prep + prep_wrap_off(W)) + w0;
+    uint32_t n = 0;
 #pragma unroll
-        for (int j = 0; j < NB / 4; ++j) {
-            const uint4 v = reinterpret_cast<const uint4 *>(code + w0)[j];
-            c[4 * j] = v.x; c[4 * j + 1] = v.y; c[4 * j + 2] = v.z; c[4 * j + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < NB; ++j) c[j] = code[w0 + j];
+    for (int j = 0; j < NWD; ++j) {
+        const uint32_t x = c[j] & wp[j];
+        n += static_cast<uint32_t>(__popc(x & (x >> 1) & (x >> 2) & (x >> 3) & 0x11111111u));
     }
-    // one accumulator per plane (six independent chains), four words at a
-    // time: the six plane reads of a group are in flight together, and the
-    // next group's reads are issued before this group's popcounts; the
-    // code's own popcount (the level offset 1) joins plane 0's chain
-    uint32_t acc[kPlanes];
+    return n;
+}
+
+// raw of NB neighbour codes per lane of WT words each.
+template <int NB, int WT>
+__device__ __forceinline__ void raw_batch(const uint32_t (&c)[NB][WT], const unsigned char *prep, bool any_wrap,
+                                          float (&raw)[NB]) {
+    v4f acc[NB];
 #pragma unroll
-    for (int p = 0; p < kPlanes; ++p) acc[p] = 0;
+    for (int b = 0; b < NB; ++b) acc[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    raw_mfma<NB, WT>(c, prep, level_rows(WT), 0, acc);
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[0] = bcnt_acc(c[j], acc[0]);
-    uint4 cur[kPlanes], nxt[kPlanes];
-#pragma unroll
-    for (int p = 0; p < kPlanes; ++p) cur[p] = reinterpret_cast<const uint4 *>(planes + p * W + w0)[0];
-#pragma unroll
-    for (int j = 0; j < NB / 4; ++j) {
-        if (j + 1 < NB / 4) {
-#pragma unroll
-            for (int p = 0; p < kPlanes; ++p) nxt[p] = reinterpret_cast<const uint4 *>(planes + p * W + w0)[j + 1];
-        }
-#pragma unroll
-        for (int p = 0; p < kPlanes; ++p) {
-            acc[p] = bcnt_acc(c[4 * j] & cur[p].x, acc[p]);
-            acc[p] = bcnt_acc(c[4 * j + 1] & cur[p].y, acc[p]);
-            acc[p] = bcnt_acc(c[4 * j + 2] & cur[p].z, acc[p]);
-            acc[p] = bcnt_acc(c[4 * j + 3] & cur[p].w, acc[p]);
-        }
-        if (j + 1 < NB / 4) {
-#pragma unroll
-            for (int p = 0; p < kPlanes; ++p) cur[p] = nxt[p];
-        }
-    }
-    // sum_p 2^p acc[p], top plane first
-    uint32_t hb = acc[kPlanes - 1];
-#pragma unroll
-    for (int p = kPlanes - 2; p >= 0; --p) hb = (hb << 1) + acc[p];
-    raw += hb;
-    if (any_zero) {
-        const uint32_t *zp = planes + kZeroPlane * W + w0;
-#pragma unroll
-        for (int j = 0; j < NB; ++j) raw -= static_cast<uint32_t>(__popc(c[j] & zp[j]));
-    }
+    for (int b = 0; b < NB; ++b) raw[b] = raw_value(acc[b]);
     if (any_wrap) {
-        const uint32_t *wp = planes + kWrapPlane * W + w0;
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const uint32_t x = c[j] & wp[j];
-            wraps += __popc(x & (x >> 1) & (x >> 2) & (x >> 3) & 0x11111111u);
-        }
+        for (int b = 0; b < NB; ++b) raw[b] -= static_cast<float>(256u * wrap_count<WT>(c[b], prep, WT, 0));
     }
 }
 
-// raw for one neighbour code of W words (W a power of two >= 8: padded
-// dimension >= 256), the same sum as raw_partial over [0, W): the code words
-// are loaded 32 at a time (eight 16-byte loads when the row layout keeps
-// codes 16-byte aligned), and each plane's matching words come from LDS as
-// 16-byte reads.
-__device__ __forceinline__ int32_t raw_words(const uint32_t *__restrict__ code, const uint32_t *planes, int W,
-                                             bool vec_ok, bool any_wrap, bool any_zero) {
-    uint32_t raw = 0, wraps = 0;
-    if (W >= 32) {
-        for (int w0 = 0; w0 < W; w0 += 32) raw_span<32>(code, planes, W, w0, vec_ok, any_wrap, any_zero, raw, wraps);
-    } else if (W == 16) {
-        raw_span<16>(code, planes, W, 0, vec_ok, any_wrap, any_zero, raw, wraps);
-    } else {
-        raw_span<8>(code, planes, W, 0, vec_ok, any_wrap, any_zero, raw, wraps);
+// NWD words from w0 of the codes of NB neighbours per lane, where `want`
+// (lane masks) asks for them; added to acc and wraps.
+template <int NB, int NWD>
+__device__ __forceinline__ void raw_span(const uint32_t *const (&code)[NB], const uint64_t (&want)[NB],
+                                         const unsigned char *prep, LevelRows lr, uint32_t W, int w0, bool vec_ok,
+                                         bool any_wrap, v4f (&acc)[NB], uint32_t (&wraps)[NB]) {
+    uint32_t c[NB][NWD];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+#pragma unroll
+        for (int j = 0; j < NWD; ++j) asm volatile("" : "=v"(c[b][j]));  // any value: see raw_words
+        if (lane_in(want[b])) {
+            if (vec_ok) {
+#pragma unroll
+                for (int j = 0; j < NWD / 4; ++j) {
+                    const uint4 v = reinterpret_cast<const uint4 *>(code[b] + w0)[j];
+                    c[b][4 * j] = v.x; c[b][4 * j + 1] = v.y; c[b][4 * j + 2] = v.z; c[b][4 * j + 3] = v.w;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NWD; ++j) c[b][j] = code[b][w0 + j];
+            }
+        }
     }
-    return static_cast<int32_t>(raw - 256u * wraps);
+    raw_mfma<NB, NWD>(c, prep, lr, w0, acc);
+    if (any_wrap) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) wraps[b] += wrap_count<NWD>(c[b], prep, W, w0);
+    }
+}
+
+// raw of NB neighbour codes per lane of W words each (W a power of two >= 8:
+// padded dimension >= 256), loaded up to NWD words at a time with 16-byte
+// loads when the row layout keeps codes 16-byte aligned.  Every lane of the
+// wave comes here (the matrix unit takes all lanes' operands).  The codes of
+// lanes outside `want` are not read: such a lane feeds whatever its registers
+// hold, which reaches its own result alone (every pattern is a finite 4-bit
+// float, and no other lane's result has a nonzero factor for it).
+template <int NB>
+__device__ __forceinline__ void raw_words(const uint32_t *const (&code)[NB], const uint64_t (&want)[NB],
+                                          const unsigned char *prep, int W, bool vec_ok, bool any_wrap,
+                                          float (&raw)[NB]) {
+    v4f acc[NB];
+    uint32_t wraps[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        acc[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        wraps[b] = 0u;
+    }
+    const LevelRows lr = level_rows(static_cast<uint32_t>(W));
+    if (W >= 32) {
+        for (int w0 = 0; w0 < W; w0 += 32) raw_span<NB, 32>(code, want, prep, lr, W, w0, vec_ok, any_wrap, acc, wraps);
+    } else if (W == 16) {
+        raw_span<NB, 16>(code, want, prep, lr, W, 0, vec_ok, any_wrap, acc, wraps);
+    } else {
+        raw_span<NB, 8>(code, want, prep, lr, W, 0, vec_ok, any_wrap, acc, wraps);
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) raw[b] = raw_value(acc[b]) - static_cast<float>(256u * wraps[b]);
 }
 
 // utils.cuh:989-993 with nvcc's contraction of the two multiply-adds.
-__device__ __forceinline__ float estimate_formula(int32_t raw, int32_t sum_q, float width, float low,
+// raw and sum_q are whole numbers below 2^18, so 2 raw - sum_q is exact.
+__device__ __forceinline__ float estimate_formula(float raw, float sum_q, float width, float low,
                                                   float tx, float fdq, float fvq, float pdist) {
-    const float rf = static_cast<float>((raw << 1) - sum_q);
+    const float rf = fmaf(2.0f, raw, -sum_q);
     float est = tx + pdist;
     est = fmaf(fdq * width, rf, est);
     est = fmaf(fvq, low, est);
@@ -1374,67 +1457,6 @@ __device__ __forceinline__ void load_code(const uint32_t *__restrict__ code, boo
     for (int w = 0; w < WT; ++w) c[w] = code[w];
 }
 
-// Horner step over the planes of WT words: 2 acc + sum_w popcount(c_w & pw_w)
-// (the top plane starts from zero).
-template <int WT>
-__device__ __forceinline__ uint32_t plane_step(const uint32_t *c, const uint32_t *pw, uint32_t acc, bool top) {
-    uint32_t a = top ? static_cast<uint32_t>(__popc(c[0] & pw[0])) : bcnt_acc(c[0] & pw[0], acc << 1);
-#pragma unroll
-    for (int w = 1; w < WT; ++w) a = bcnt_acc(c[w] & pw[w], a);
-    return a;
-}
-
-// raw for NB code blocks at once, walking the planes one at a time from LDS
-// (one plane's WT words live at a time), top plane first: raw_b =
-// popcount(code_b) + sum_p 2^p popcount(code_b & plane_p) (the planes hold
-// q - 1) - popcount(code_b & zero plane) - 256 * wraps_b, the powers of two
-// by Horner's rule (one shift per plane and block).
-template <int NB, int WT>
-__device__ __forceinline__ void raw_batch(const uint32_t (&c)[NB][WT], const uint32_t *planes, bool any_wrap,
-                                          bool any_zero, int32_t (&raw)[NB]) {
-    uint32_t acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = 0;
-#pragma unroll
-    for (int p = kPlanes - 1; p >= 0; --p) {
-        uint32_t pw[WT];
-#pragma unroll
-        for (int w = 0; w < WT; ++w) pw[w] = planes[p * WT + w];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b] = plane_step<WT>(c[b], pw, acc[b], p == kPlanes - 1);
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int w = 0; w < WT; ++w) acc[b] = bcnt_acc(c[b][w], acc[b]);
-    if (any_zero) {
-        uint32_t pw[WT];
-#pragma unroll
-        for (int w = 0; w < WT; ++w) pw[w] = planes[kZeroPlane * WT + w];
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int w = 0; w < WT; ++w) acc[b] -= static_cast<uint32_t>(__popc(c[b][w] & pw[w]));
-    }
-    if (any_wrap) {
-        uint32_t pw[WT];
-#pragma unroll
-        for (int w = 0; w < WT; ++w) pw[w] = planes[kWrapPlane * WT + w];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            uint32_t wr = 0;
-#pragma unroll
-            for (int w = 0; w < WT; ++w) {
-                const uint32_t x = c[b][w] & pw[w];
-                wr += __popc(x & (x >> 1) & (x >> 2) & (x >> 3) & 0x11111111u);
-            }
-            acc[b] -= 256u * wr;
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) raw[b] = static_cast<int32_t>(acc[b]);
-}
-
 // One pass of exact distances over children e0 .. e0 + 2 PB - 1 (child
 // e0 + 2 j + h on half h): PB row loads per lane issued together, then a
 // reduce-scatter over the half.  At distance 16 lanes keep children
@@ -1599,48 +1621,76 @@ __device__ __forceinline__ void exact_batch(const SearchParams &P, const G &g, i
     exact_batch_range<DPL>(P, g, 0, n, slot_list, cd, ci, qr, qv);
 }
 
-// The keep_k smallest valid (value, lane) pairs of each 32-lane half, as
-// warp_keep_topk_smallest_f32 (utils.cuh:251-267) selects them, found by
-// keep_k rounds of group argmin (G = 32: half-wave; 16: 16-lane row) instead
-// of a 32-step rank count.  keep_k is uniform within each group; valid lanes
-// and the result are lane masks.
+// Group t's bits of a lane mask (G lanes each), left at their place in the
+// 32-bit half that holds them, and the mask of all groups.
 template <int G>
-__device__ __forceinline__ uint64_t select_smallest(float value, uint64_t valid, int keep_k, int max_k) {
-    // order-preserving unsigned image of the float; -0 joins +0 so equal
-    // values tie exactly as in the float comparison
-    const uint32_t bits = __float_as_uint(value == 0.0f ? 0.0f : value);
-    const uint32_t key = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
-    uint64_t remaining = valid, kept = 0ull;
-    for (int r = 0; r < max_k; ++r) {
-        uint32_t m = lane_in(remaining) ? key : 0xFFFFFFFFu;
-        // minimum over the 32-lane half: quad (xor 1, xor 2), then the
-        // half-row and row mirrors bring in the other quad and the other
-        // half-row, then the neighbouring row
-        m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0xB1, 0xF, 0xF, true)));
-        m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0x4E, 0xF, 0xF, true)));
-        m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0x141, 0xF, 0xF, true)));
-        m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0x140, 0xF, 0xF, true)));
-        if constexpr (G == 32) m = min16(m);  // (G = 16: the row's minimum is the group's)
-        // the lowest lane of each group holding its group's minimum (x & -x on
-        // each G-bit part of the mask), taken while the group keeps more
-        const uint64_t cand = ballot(key == m) & remaining;
-        uint64_t first;
-        if constexpr (G == 32) {
-            const uint32_t c0 = static_cast<uint32_t>(cand), c1 = static_cast<uint32_t>(cand >> 32);
-            first = (static_cast<uint64_t>(c1 & (0u - c1)) << 32) | (c0 & (0u - c0));
-        } else {
-            first = 0ull;
+__device__ __forceinline__ uint32_t group_bits(uint64_t m, int t) {
+    const uint32_t half = static_cast<uint32_t>(m >> (G * t >= 32 ? 32 : 0));
+    return G == 32 ? half : half & (t & 1 ? 0xFFFF0000u : 0x0000FFFFu);
+}
+template <int G>
+__device__ __forceinline__ uint64_t group_join(const uint32_t (&b)[64 / G]) {
+    if constexpr (G == 32) return static_cast<uint64_t>(b[1]) << 32 | b[0];
+    else return static_cast<uint64_t>(b[2] | b[3]) << 32 | (b[0] | b[1]);
+}
+
+// One step of select_smallest for one sub-round: the lowest lane of each
+// group that holds the group's smallest remaining key, taken where the group
+// keeps more than r.
+template <int G>
+__device__ __forceinline__ void select_step(uint32_t key, int r, const int (&rounds)[64 / G], uint32_t (&rest)[64 / G],
+                                            uint32_t (&kept)[64 / G]) {
+    const uint64_t remaining = group_join<G>(rest);
+    uint32_t m = lane_in(remaining) ? key : 0xFFFFFFFFu;
+    // minimum over the group: quad (xor 1, xor 2), then the half-row and row
+    // mirrors bring in the other quad and the other half-row, then the
+    // neighbouring row
+    m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0xB1, 0xF, 0xF, true)));
+    m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0x4E, 0xF, 0xF, true)));
+    m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0x141, 0xF, 0xF, true)));
+    m = min(m, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(m), 0x140, 0xF, 0xF, true)));
+    if constexpr (G == 32) m = min16(m);  // (G = 16: the row's minimum is the group's)
+    const uint64_t cand = ballot(key == m) & remaining;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const uint32_t c = static_cast<uint32_t>(cand >> (16 * g)) & 0xFFFFu;
-                first |= static_cast<uint64_t>(c & (0u - c)) << (16 * g);
-            }
-        }
-        const uint64_t take = first & ballot(r < keep_k);
-        kept |= take;
-        remaining &= ~take;
+    for (int t = 0; t < 64 / G; ++t) {
+        const uint32_t c = group_bits<G>(cand, t);
+        const uint32_t take = r < rounds[t] ? c & (0u - c) : 0u;
+        kept[t] |= take;
+        rest[t] &= ~take;
     }
-    return kept;
+}
+
+// Adds to kept the rounds[s][t] smallest (value, lane) pairs among the lanes
+// rest[s][t] of each G-lane group t of NS sub-rounds, as
+// warp_keep_topk_smallest_f32 (utils.cuh:251-267) selects them, found by
+// rounds of group argmin (G = 32: half-wave; 16: 16-lane row) instead of a
+// 32-step rank count.  The first round, all that most groups need, runs on
+// every sub-round at once: its cross-lane steps are a chain, and the
+// sub-rounds' chains fill each other's gaps.  maxk is the largest of rounds.
+template <int G, int NS>
+__device__ __forceinline__ void select_smallest(const float (&value)[NS], uint32_t (&rest)[NS][64 / G],
+                                                const int (&rounds)[NS][64 / G], int maxk,
+                                                uint32_t (&kept)[NS][64 / G]) {
+    if (maxk == 0) return;
+    uint32_t key[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        // order-preserving unsigned image of the float; -0 joins +0 so equal
+        // values tie exactly as in the float comparison
+        const uint32_t bits = __float_as_uint(value[s] + 0.0f);
+        key[s] = bits ^ (static_cast<uint32_t>(static_cast<int32_t>(bits) >> 31) | 0x80000000u);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) select_step<G>(key[s], 0, rounds[s], rest[s], kept[s]);
+    if (maxk == 1) return;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        int k = 0;
+#pragma unroll
+        for (int t = 0; t < 64 / G; ++t) k = max(k, rounds[s][t]);
+#pragma unroll 1
+        for (int r = 1; r < k; ++r) select_step<G>(key[s], r, rounds[s], rest[s], kept[s]);
+    }
 }
 
 // Visited test for up to four keys per lane: both buckets of every key are
@@ -1706,8 +1756,8 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
 // a sixth), which LDS also allows for beams up to 256 (6,144 bytes a
 // workgroup at beam 256).  The generic-geometry instantiation (padded dimension
 // >= 256) gets 3 (<= 168 VGPRs) for its wide code batches and the plane reads
-// it keeps in flight: at padded dimension 2048 its LDS (raw query, planes,
-// rotation scratch) holds it to 3 waves per SIMD anyway, and at 1024 a
+// it keeps in flight: at padded dimension 2048 its LDS (digit rows, rotation
+// scratch) holds it to 3 waves per SIMD anyway, and at 1024 a
 // 1,000-query launch fills one wave per SIMD.
 // NW = 2: the team form (two waves per query; see TeamBlock).  Wave 0 leads:
 // it runs every phase, the helper wave joins it in stage II's rounds and the
@@ -1748,18 +1798,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
     // (the same layout function the host sizes the launch with)
     constexpr bool kFixedGeo = Geo<DIM_T, DEG_T>::kFixed;
     constexpr LdsLayout kL = lds_layout(DIM_T, Geo<DIM_T, DEG_T>::kB, 0, 0);
-    const uint32_t plane_off = kFixedGeo ? kL.plane_off : P.lds.plane_off;
+    const uint32_t msort_off = kFixedGeo ? kL.msort_off : P.lds.msort_off;
     const uint32_t scratch_off = kFixedGeo ? kL.scratch_off : P.lds.scratch_off;
     const uint32_t prof_off = P.lds.prof_off;
-    static_assert(kL.msort_off == 0u, "fixed LDS regions");
+    static_assert(kL.prep_off == 0u, "fixed LDS regions");
     uint32_t *H = reinterpret_cast<uint32_t *>(smem + P.lds.hash_off);
     // beam pairs: bp[-1] and bp[pbeam] are sentinels
     uint2 *bp = reinterpret_cast<uint2 *>(smem + P.lds.beam_off) + 1;
-    uint2 *ms = reinterpret_cast<uint2 *>(smem + kL.msort_off) + 1;
+    uint2 *ms = reinterpret_cast<uint2 *>(smem + msort_off) + 1;
     // candidate slot s: distance at cd[2 s], id at ci[2 s] (the pair ms[s])
     float *cd = reinterpret_cast<float *>(ms);
     uint32_t *ci = reinterpret_cast<uint32_t *>(ms) + 1;
-    uint32_t *planes = reinterpret_cast<uint32_t *>(smem + plane_off);
+    unsigned char *prep = smem + kL.prep_off;
+    uint32_t *prep_w = reinterpret_cast<uint32_t *>(prep);
     uint32_t *alist = reinterpret_cast<uint32_t *>(smem + scratch_off);
     uint32_t *pnode = alist + 32;
     float *pdist = reinterpret_cast<float *>(pnode + 8);
@@ -1771,9 +1822,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
         t_last = __builtin_amdgcn_s_memtime();
     }
 
-    // ---- query preparation (the visited table's LDS holds the rotation); a
-    // query resumed by the second slice reads back the planes and constants
-    // the first slice kept instead
+    // ---- query preparation (the beam's and the table's LDS hold the rotation); a
+    // query resumed by the second slice reads back the prepared query the
+    // first slice kept instead
     float qlow = 0.0f, qhigh = 0.0f, qwidth = 0.0f;
     int sum_q = 0;
     const bool resuming = kSliceable && P.slice_resume > 0;
@@ -1782,14 +1833,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             const uint32_t *sp = P.slice_state + kSliceHeader +
                                  static_cast<uint64_t>(qid) * slice_words(static_cast<uint32_t>(P.pbeam), B) +
                                  slice_prep_offset(static_cast<uint32_t>(P.pbeam));
-            for (int i = lane; i < 8 * W; i += 64) planes[i] = sp[4 + i];
+            for (int i = lane; i < static_cast<int>(prep_words(W)); i += 64) prep_w[i] = sp[4 + i];
             qlow = __uint_as_float(uni(sp[0]));
             qwidth = __uint_as_float(uni(sp[1]));
             sum_q = static_cast<int>(uni(sp[2]));
             lead_sync<NW>();
         } else {
             prepare_query<NW>(P.queries + static_cast<uint64_t>(qid) * g.dim, P.signs, g.dim, B,
-                              reinterpret_cast<float *>(H), nullptr, planes, qlow, qhigh, qwidth, sum_q, nullptr);
+                              reinterpret_cast<float *>(smem + P.lds.beam_off), nullptr, prep_w, qlow, qhigh, qwidth, sum_q, nullptr);
         }
     }
     // the query is read from global memory, where it stays cached (the
@@ -1799,27 +1850,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
     constexpr int WTR = WT > 0 ? WT : 1;
     // whether any chunk of the quantized query wraps the reference's uint8
     // LUT entry (then the estimates subtract the wrapped chunks)
-    uint32_t any_wrap = 0u, any_zero = 0u;  // 0 / 1 (sflag at each use)
-    if (lead) {
-        if constexpr (WT > 0) {
-            uint32_t wor = 0, zor = 0;
-#pragma unroll
-            for (int w = 0; w < WT; ++w) {
-                wor |= planes[kWrapPlane * WT + w];
-                zor |= planes[kZeroPlane * WT + w];
-            }
-            any_wrap = uni(wor) != 0u ? 1u : 0u;
-            any_zero = uni(zor) != 0u ? 1u : 0u;
-        } else {
-            uint32_t wor = 0, zor = 0;
-            for (int w = lane; w < W; w += 64) {
-                wor |= planes[kWrapPlane * W + w];
-                zor |= planes[kZeroPlane * W + w];
-            }
-            any_wrap = any_lane(wor != 0u) ? 1u : 0u;
-            any_zero = any_lane(zor != 0u) ? 1u : 0u;
-        }
-    }
+    uint32_t any_wrap = 0u;  // 0 / 1 (sflag at each use)
+    if (lead) any_wrap = wraps_anywhere(prep, W);
     constexpr int DPLR = DPL > 0 ? DPL : 1;
     float qr[DPLR];
 #pragma unroll
@@ -1855,7 +1887,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             tb->qwidth_bits = __float_as_uint(qwidth);
             tb->qlow_bits = __float_as_uint(qlow);
             tb->any_wrap = any_wrap;
-            tb->any_zero = any_zero;
         }
         __syncthreads();
         if (!lead) {
@@ -1863,10 +1894,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             qwidth = __uint_as_float(uni(tb->qwidth_bits));
             qlow = __uint_as_float(uni(tb->qlow_bits));
             any_wrap = uni(tb->any_wrap) != 0u ? 1u : 0u;
-            any_zero = uni(tb->any_zero) != 0u ? 1u : 0u;
         }
     }
 
+    const float sumq_f = static_cast<float>(sum_q);
     Controller ctl{1, kPhase1Rho, 0, kMaxIndex, 0, false, entry_d, FLT_MAX, FLT_MAX, uni(entry_guard(entry_d))};
     uint32_t c_iters = 0, c_exp = 0, c_ids = 0, c_est = 0, c_exact = 1, c_st2 = kMaxIndex;
     const int beam_sz = P.beam, pbeam = P.pbeam;
@@ -2117,17 +2148,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                     FG_COUNT(c_est += static_cast<uint32_t>(valid_count));
                     const uint32_t *codes = reinterpret_cast<const uint32_t *>(prow + g.code);
                     const bool valid = child != kMaxIndex;
-                    float est = FLT_MAX;
-                    int32_t r1[1] = {0};
+                    // computed on every lane, selected for the valid ones
+                    float r1[1];
                     if constexpr (WT > 0) {
-                        // computed on every lane, selected for the valid ones
-                        raw_batch<1, WT>(c1, planes, sflag(any_wrap), sflag(any_zero), r1);
-                        est = tx == FLT_MAX ? 0.0f : estimate_formula(r1[0], sum_q, qwidth, qlow, tx, fdq, fvq, pd0);
-                    } else if (valid) {
-                        const int32_t raw = raw_words(codes + static_cast<uint64_t>(nsafe) * W, planes, W, vec_ok,
-                                                      sflag(any_wrap), sflag(any_zero));
-                        est = tx == FLT_MAX ? 0.0f : estimate_formula(raw, sum_q, qwidth, qlow, tx, fdq, fvq, pd0);
+                        raw_batch<1, WT>(c1, prep, sflag(any_wrap), r1);
+                    } else {
+                        const uint32_t *const code1[1] = {codes + static_cast<uint64_t>(nsafe) * W};
+                        const uint64_t want1[1] = {ballot(valid)};
+                        raw_words<1>(code1, want1, prep, W, vec_ok, sflag(any_wrap), r1);
                     }
+                    const float est =
+                        tx == FLT_MAX ? 0.0f : estimate_formula(r1[0], sumq_f, qwidth, qlow, tx, fdq, fvq, pd0);
                     const bool fin = isfinite(est);
                     child = (valid && !fin) ? kMaxIndex : child;
                     dist = valid ? (fin ? est : FLT_MAX) : dist;
@@ -2200,7 +2231,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 const int sr0 = wv * SRN;
                 uint32_t cid[SRN];
                 bool val[SRN];
-                int an[SRN], tsk[SRN], pix[SRN];
+                int pix[SRN];
                 const float *prw[SRN];
                 uint32_t rof[SRN];  // fixed geometry: the parents' row byte offsets
                 float tx[SRN], fdq[SRN], fvq[SRN];
@@ -2217,12 +2248,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 for (int sr = 0; sr < SRN; ++sr) {
                     const int task = rbase + TPW * (sr0 + sr) + grp;
                     const bool tact = task < tasks;
-                    const int pidx = tact ? task / tiles : 0;
-                    const int tile = tact ? task - pidx * tiles : 0;
+                    int pidx = tact ? task : 0, tile = 0;
+                    if (tiles > 1) {
+                        pidx = tact ? task / tiles : 0;
+                        tile = tact ? task - pidx * tiles : 0;
+                    }
                     const int nidx = tile * 32 + nlg;
                     lact[sr] = tact && nidx < deg;
                     nsafe[sr] = nidx < deg ? nidx : deg - 1;
-                    tsk[sr] = tact ? tile * 32 : -1;
                     pix[sr] = pidx;
                     if constexpr (kFixedGeo) {
                         rof[sr] = __umul24(pnode[pidx], Geo<DIM_T, DEG_T>::kRowB);
@@ -2231,8 +2264,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                         prw[sr] = data + static_cast<uint64_t>(pnode[pidx]) * g.row;
                         cid[sr] = reinterpret_cast<const uint32_t *>(prw[sr] + g.nbr)[nsafe[sr]];
                     }
-                    int a = tact ? deg - tile * 32 : 0;
-                    an[sr] = a > 32 ? 32 : a;
                     FG_COUNT(c_ids += static_cast<uint32_t>(__popcll(ballot(lact[sr]))));
                 }
 #pragma unroll
@@ -2273,74 +2304,109 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
 #pragma unroll
                 for (int sr = 0; sr < SRN; ++sr) val[sr] = cid[sr] != kMaxIndex && cid[sr] < np32;
                 hash_contains_n<SRN>(H, nbk, cid, val);
-                // (c) which tasks need estimates.  Lane predicates from here on
-                // are masks taken straight from compares.  A task without
-                // children has no valid lane, so it never needs estimates and
-                // its keep limit is never read.
-                uint64_t valm[SRN], needm[SRN];
-                int keep[SRN];
+                // (c) which tasks need estimates.  From here on predicates are
+                // lane masks taken straight from compares, and each task works
+                // on its own bits of them with scalar instructions, beside the
+                // other waves' vector ones.  need: all ones or zero.
+                uint64_t valm[SRN];
+                int lim[SRN][TPW];
+                uint32_t need[SRN][TPW];
 #pragma unroll
                 for (int sr = 0; sr < SRN; ++sr) {
                     valm[sr] = ballot(val[sr]);
-                    const int rvc = static_cast<int>(group_popc<G>(valm[sr]));
-                    keep[sr] = an[sr] == an_full ? lim_full : lim_last;
-                    needm[sr] = ballot(keep[sr] < rvc);
-                    FG_COUNT(c_est += static_cast<uint32_t>(__popcll(needm[sr] & valm[sr])));
+#pragma unroll
+                    for (int t = 0; t < TPW; ++t) {
+                        lim[sr][t] = lim_full;
+                        if (lim_last != lim_full && (rbase + TPW * (sr0 + sr) + t) % tiles == tiles - 1)
+                            lim[sr][t] = lim_last;
+                        need[sr][t] = lim[sr][t] < __popc(group_bits<G>(valm[sr], t)) ? ~0u : 0u;
+                        FG_COUNT(c_est += static_cast<uint32_t>(__popc(need[sr][t] & group_bits<G>(valm[sr], t))));
+                    }
                 }
                 FG_PHASE(6);
                 // (d) estimates, kth-near counts, keep decisions
+                float raw[SRN], est[SRN];
+                if constexpr (WT > 0) {
+                    // (two sub-rounds at a time: four at once would hold eight
+                    // more registers, and with them the sixth wave per SIMD)
+                    constexpr int NB = SRN > 2 ? 2 : SRN;
+#pragma unroll
+                    for (int s2 = 0; s2 < SRN; s2 += NB) {
+                        uint32_t c2[NB][WT];
+                        float r[NB];
+#pragma unroll
+                        for (int b = 0; b < NB; ++b)
+#pragma unroll
+                            for (int w = 0; w < WT; ++w) c2[b][w] = code[s2 + b][w];
+                        raw_batch<NB, WT>(c2, prep, sflag(any_wrap), r);
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) raw[s2 + b] = r[b];
+                    }
+                } else {
+                    // two sub-rounds share each read of the query's rows
+                    constexpr int NB = SRN > 1 ? 2 : 1;
+#pragma unroll
+                    for (int s2 = 0; s2 < SRN; s2 += NB) {
+                        const uint32_t *cp[NB];
+                        uint64_t want[NB], any = 0ull;
+                        float r[NB];
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) {
+                            cp[b] = reinterpret_cast<const uint32_t *>(prw[s2 + b] + g.code) +
+                                    static_cast<uint64_t>(nsafe[s2 + b]) * W;
+                            want[b] = group_join<G>(need[s2 + b]) & valm[s2 + b];  // (G is 32 here)
+                            any |= want[b];
+                            r[b] = 0.0f;
+                        }
+                        if (any != 0ull) raw_words<NB>(cp, want, prep, W, vec_ok, sflag(any_wrap), r);
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) raw[s2 + b] = r[b];
+                    }
+                }
                 uint64_t klm[SRN];
-                int32_t rawb[SRN];
-                if constexpr (WT > 0) raw_batch<SRN, WT>(code, planes, sflag(any_wrap), sflag(any_zero), rawb);
+                uint32_t rest[SRN][TPW], kept[SRN][TPW];
+                int rounds[SRN][TPW], maxk = 0;
+                const float cutoff = kth_valid ? kth : -INFINITY;
 #pragma unroll
                 for (int sr = 0; sr < SRN; ++sr) {
-                    float est = FLT_MAX;
-                    const uint64_t scored = needm[sr] & valm[sr];
-                    if constexpr (WT > 0) {
-                        // computed on every lane and selected (most lanes need it;
-                        // a branch would cost more than the few wasted lanes)
-                        const float e = estimate_formula(rawb[sr], sum_q, qwidth, qlow, tx[sr], fdq[sr], fvq[sr],
-                                                         pdist[pix[sr]]);
-                        est = (lane_in(scored) && tx[sr] != FLT_MAX) ? e : FLT_MAX;
-                    } else if (lane_in(scored) && tx[sr] != FLT_MAX) {
-                        const int nidx = tsk[sr] + nlg;
-                        const int32_t raw = raw_words(reinterpret_cast<const uint32_t *>(prw[sr] + g.code) +
-                                                          static_cast<uint64_t>(nidx) * W,
-                                                      planes, W, vec_ok, sflag(any_wrap), sflag(any_zero));
-                        est = estimate_formula(raw, sum_q, qwidth, qlow, tx[sr], fdq[sr], fvq[sr], pdist[pix[sr]]);
-                    }
+                    // computed on every lane (most need it); a lane whose task
+                    // needs no estimates is kept by its mask alone
+                    const float e = estimate_formula(raw[sr], sumq_f, qwidth, qlow, tx[sr], fdq[sr], fvq[sr],
+                                                     pdist[pix[sr]]);
+                    est[sr] = tx[sr] != FLT_MAX ? e : FLT_MAX;
                     // a scored child with a non-finite estimate is dropped
                     // (finiteness as an integer compare on opaque bits, which
                     // the ballot takes as it is; a float class test would pass
                     // through a vector register on its way to the mask)
-                    uint32_t eb = __float_as_uint(est);
+                    uint32_t eb = __float_as_uint(est[sr]);
                     asm volatile("" : "+v"(eb));
                     const uint64_t finm = ballot((eb & 0x7F800000u) != 0x7F800000u);
-                    valm[sr] = (valm[sr] & ~scored) | (scored & finm);
-                    uint64_t kl = valm[sr];
-                    if (needm[sr] != 0ull) {
-                        const uint64_t belowm = kth_valid ? (valm[sr] & ballot(est <= kth)) : 0ull;
-                        const uint32_t near = group_popc<G>(belowm);
-                        const int kp = keep[sr];
-                        const bool nd = lane_in(needm[sr]);
-                        const int eff = nd ? keep_with_cutoff(kp, kth_valid, near) : kp;
+                    // (no estimate lies at or below -infinity: without a valid
+                    // cutoff nothing is near)
+                    const uint64_t nearm = ballot(est[sr] <= cutoff) & finm & valm[sr];
+#pragma unroll
+                    for (int t = 0; t < TPW; ++t) {
+                        const uint32_t nd = need[sr][t], below = group_bits<G>(nearm, t) & nd;
+                        const int near = __popc(below);
                         // With a valid cutoff and 1 <= near <= keep the count is
                         // near, and the near smallest (value, lane) pairs are the
                         // ones at or below the cutoff: every such lane ranks
                         // ahead of every lane above it.  No selection rounds.
-                        const uint64_t cutm =
-                            kth_valid ? (needm[sr] & ballot(near >= 1u) & ballot(static_cast<int>(near) <= kp)) : 0ull;
-                        const int rounds = (nd && !lane_in(cutm)) ? eff : 0;
-                        // uniform within each group: the largest over the groups' first lanes
-                        int maxk = max(__builtin_amdgcn_readlane(rounds, 0), __builtin_amdgcn_readlane(rounds, 32));
-                        if constexpr (G == 16)
-                            maxk = max(maxk, max(__builtin_amdgcn_readlane(rounds, 16), __builtin_amdgcn_readlane(rounds, 48)));
-                        const uint64_t selm = select_smallest<G>(est, valm[sr], eff, maxk);
-                        const uint64_t effm = ballot(eff > 0);
-                        kl = (valm[sr] & ~needm[sr]) | (needm[sr] & valm[sr] & effm & ((cutm & belowm) | (selm & ~cutm)));
+                        // Otherwise keep_with_cutoff's count: one for near = 0
+                        // with a valid cutoff, else the limit.
+                        int k = near > lim[sr][t] ? lim[sr][t] : 0;
+                        k = near == 0 ? (kth_valid ? 1 : lim[sr][t]) : k;
+                        k &= static_cast<int>(nd);
+                        rounds[sr][t] = k;
+                        maxk = max(maxk, k);
+                        const uint32_t v = group_bits<G>(valm[sr], t);
+                        rest[sr][t] = v & group_bits<G>(finm, t);
+                        kept[sr][t] = (v & ~nd) | (k == 0 ? below : 0u);
                     }
-                    klm[sr] = kl;
                 }
+                select_smallest<G, SRN>(est, rest, rounds, maxk, kept);
+#pragma unroll
+                for (int sr = 0; sr < SRN; ++sr) klm[sr] = group_join<G>(kept[sr]);
                 // the kept lanes of all sub-rounds; in the team form the
                 // helper's half reaches the lead wave through LDS
                 uint64_t klmA[SR];
@@ -2372,16 +2438,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 if (lead) {
                     // (e) kept children listed in (task, lane) order
                     uint32_t total = 0;
+                    const uint32_t list_spare =
+                        (P.lds.beam_off + 8u * static_cast<uint32_t>(pbeam + 3) - scratch_off) / 4u;
 #pragma unroll
                     for (int sr = 0; sr < SR; ++sr) {
                         // the sub-round's TPW tasks sit in lane order and follow
                         // each other in the list: a kept lane's place is the running
                         // total plus its rank among the kept lanes of the wave
-                        if (lane_in(klmA[sr])) {
-                            const uint32_t e = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(klmA[sr] >> 32),
-                                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(klmA[sr]), total));
-                            if (e < 32) alist[e] = cidA[sr];
-                        }
+                        // (a lane with nothing to list, and one past the 32nd
+                        // place, writes the beam's pad entry that takes the
+                        // merge's unused slots: no branch)
+                        const uint32_t e = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(klmA[sr] >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(klmA[sr]), total));
+                        alist[(lane_in(klmA[sr]) & (e < 32u)) ? e : list_spare] = cidA[sr];
                         total += static_cast<uint32_t>(__popcll(klmA[sr]));
                     }
                     lead_sync<NW>();
@@ -2468,7 +2537,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 const float kd = pair_key(bp[0]);
                 for (int i = lane; i < pbeam + 32; i += 64) sb[i] = i < pbeam ? bp[i] : ms[i - pbeam];
                 uint32_t *sp = st + slice_prep_offset(pbeam);
-                for (int i = lane; i < 8 * W; i += 64) sp[4 + i] = planes[i];
+                for (int i = lane; i < static_cast<int>(prep_words(W)); i += 64) sp[4 + i] = prep_w[i];
                 if (lane == 0) {
                     sp[0] = __float_as_uint(qlow);
                     sp[1] = __float_as_uint(qwidth);

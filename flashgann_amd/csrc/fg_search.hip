@@ -12,10 +12,10 @@
 //   * the reference's 32-lane sorting networks are data-oblivious, so the
 //     same compare-exchange sequence is replayed on the wave (two 32-lane
 //     halves, or 1-2 positions per lane) and ties resolve identically;
-//   * RaBitQ scores come from 6 popcount bit-planes of the quantized query
-//     minus one, held in LDS (raw = popcount(code) + sum_p 2^p
-//     popcount(code & plane_p)), corrected for the reference's uint8 LUT wrap,
-//     instead of per-nibble LUT gathers;
+//   * RaBitQ scores come from the matrix unit: the quantized query's levels
+//     as rows of base-4 digits times the code bits, both as 4-bit floats
+//     (raw_mfma), corrected for the reference's uint8 LUT wrap, instead of
+//     per-nibble LUT gathers;
 //   * exact distances keep the reference's per-lane accumulation order and
 //     reduction tree, so results are bitwise equal to the 32-lane original.
 // Determinism: where the reference races (concurrent inserts of one child by
@@ -275,10 +275,10 @@ __global__ __launch_bounds__(64) void fg_prepare_kernel(const float *queries, co
     const int qid = blockIdx.x;
     if (qid >= nq) return;
     float *rot = reinterpret_cast<float *>(smem);
-    uint32_t *planes = reinterpret_cast<uint32_t *>(smem + scratch_off);
+    uint32_t *prep = reinterpret_cast<uint32_t *>(smem + scratch_off);
     float lo, hi, w;
     int s;
-    prepare_query(queries + static_cast<uint64_t>(qid) * dim, signs, dim, B, rot, nullptr, planes, lo, hi, w, s,
+    prepare_query(queries + static_cast<uint64_t>(qid) * dim, signs, dim, B, rot, nullptr, prep, lo, hi, w, s,
                   quant + static_cast<uint64_t>(qid) * B);
     for (int i = lane_id(); i < B; i += 64) rotated[static_cast<uint64_t>(qid) * B + i] = rot[i];
     if (lane_id() == 0) {
@@ -296,7 +296,7 @@ struct ScoreParams {
     uint64_t row_offset, code_offset, factor_offset, npoints;
     int dim, B, deg, use_ip;
     uint32_t n;
-    uint32_t plane_off, query_off;
+    uint32_t prep_off, query_off, level_off;
 };
 
 // One workgroup per scored edge: prepares the query, then evaluates both
@@ -309,11 +309,12 @@ __global__ __launch_bounds__(64) void fg_score_kernel(ScoreParams S) {
     const int nl = lane & 31, h = lane >> 5;
     float *rot = reinterpret_cast<float *>(smem);
     float *qv = reinterpret_cast<float *>(smem + S.query_off);
-    uint32_t *planes = reinterpret_cast<uint32_t *>(smem + S.plane_off);
+    unsigned char *prep = smem + S.prep_off;
+    uint8_t *levels = smem + S.level_off;
     float lo, hi, w;
     int sq;
-    prepare_query(S.queries + static_cast<uint64_t>(S.qix[e]) * S.dim, S.signs, S.dim, S.B, rot, qv, planes, lo, hi,
-                  w, sq, nullptr);
+    prepare_query(S.queries + static_cast<uint64_t>(S.qix[e]) * S.dim, S.signs, S.dim, S.B, rot, qv,
+                  reinterpret_cast<uint32_t *>(prep), lo, hi, w, sq, levels);
     const uint32_t parent = S.parents[e];
     const int slot = static_cast<int>(S.slots[e]);
     const float *prow = S.data + static_cast<uint64_t>(parent) * S.row_offset;
@@ -322,38 +323,39 @@ __global__ __launch_bounds__(64) void fg_score_kernel(ScoreParams S) {
     const uint32_t *code = reinterpret_cast<const uint32_t *>(prow + S.code_offset) + static_cast<uint64_t>(slot) * W;
     const float *f = prow + S.factor_offset;
     const float tx = f[slot], fdq = f[S.deg + slot], fvq = f[2 * S.deg + slot];
-    // both halves split the words (theta == 1 layout) and one lane does all
-    // words (theta > 1 layout): the integer sums must agree.
-    const int hw = W >> 1;
-    const int32_t part = raw_partial(code, h * hw, (h + 1) * hw, planes, W);
-    const int32_t raw_split = add32i(part);
-    // the search kernel's own routines: raw_batch for padded dimensions 64 and
-    // 128 (W = 2, 4; the fixed geometries), raw_words for W >= 8
-    const bool vec_ok = S.row_offset % 4 == 0 && S.code_offset % 4 == 0;
-    uint32_t wor = 0, zor = 0;
-    for (int w = 0; w < W; ++w) {
-        wor |= planes[kWrapPlane * W + w];
-        zor |= planes[kZeroPlane * W + w];
-    }
-    const bool any_wrap = uni(wor) != 0u, any_zero = uni(zor) != 0u;
-    int32_t raw_full;
-    if (W == 4 || W == 2) {
-        int32_t r[1];
-        if (W == 4) {
-            uint32_t c[1][4];
-            load_code<4>(code, vec_ok, c[0]);
-            raw_batch<1, 4>(c, planes, any_wrap, any_zero, r);
-        } else {
-            uint32_t c[1][2];
-            load_code<2>(code, vec_ok, c[0]);
-            raw_batch<1, 2>(c, planes, any_wrap, any_zero, r);
+    // the levels summed chunk by chunk, each chunk's sum taken mod 256 as the
+    // reference's uint8 LUT entry is (utils.cuh:909-917, 976-980), the halves
+    // splitting the words (theta == 1 layout); and the search kernel's own
+    // routines on all words (theta > 1 layout): the integer sums must agree.
+    int32_t part = 0;
+    for (int wd = h * (W >> 1); wd < (h + 1) * (W >> 1); ++wd) {
+        const uint32_t c = code[wd];
+        for (int k = 0; k < 8; ++k) {
+            uint32_t sum = 0;
+            for (int d = 0; d < 4; ++d) sum += ((c >> (4 * k + 3 - d)) & 1u) * levels[32 * wd + 4 * k + d];
+            part += static_cast<int32_t>(sum & 255u);
         }
-        raw_full = r[0];
-    } else {
-        raw_full = raw_words(code, planes, W, vec_ok, any_wrap, any_zero);
     }
-    const float el = tx == FLT_MAX ? 0.0f : estimate_formula(raw_split, sq, w, lo, tx, fdq, fvq, pd);
-    const float es = tx == FLT_MAX ? FLT_MAX : estimate_formula(raw_full, sq, w, lo, tx, fdq, fvq, pd);
+    const float raw_split = static_cast<float>(add32i(part));
+    const bool vec_ok = S.row_offset % 4 == 0 && S.code_offset % 4 == 0;
+    const bool any_wrap = wraps_anywhere(prep, W) != 0u;
+    float r[1];
+    if (W == 4) {
+        uint32_t c[1][4];
+        load_code<4>(code, vec_ok, c[0]);
+        raw_batch<1, 4>(c, prep, any_wrap, r);
+    } else if (W == 2) {
+        uint32_t c[1][2];
+        load_code<2>(code, vec_ok, c[0]);
+        raw_batch<1, 2>(c, prep, any_wrap, r);
+    } else {
+        const uint32_t *const cp[1] = {code};
+        const uint64_t all[1] = {~0ull};
+        raw_words<1>(cp, all, prep, W, vec_ok, any_wrap, r);
+    }
+    const float raw_full = r[0], sqf = static_cast<float>(sq);
+    const float el = tx == FLT_MAX ? 0.0f : estimate_formula(raw_split, sqf, w, lo, tx, fdq, fvq, pd);
+    const float es = tx == FLT_MAX ? FLT_MAX : estimate_formula(raw_full, sqf, w, lo, tx, fdq, fvq, pd);
     const uint32_t child = reinterpret_cast<const uint32_t *>(prow + (S.factor_offset + 3 * S.deg))[slot];
     const bool child_ok = child < S.npoints;
     const float ex = uni(half_distance(S.data + static_cast<uint64_t>(child_ok ? child : 0u) * S.row_offset, qv,
@@ -1088,7 +1090,7 @@ int fg_query_prepare(fg_index *ix, const float *queries, uint32_t nq, float *rot
     if (rc == FG_OK && hipMemcpy(dq, queries, qb, hipMemcpyHostToDevice) != hipSuccess) rc = fail(FG_EDEVICE, "upload");
     if (rc == FG_OK) {
         const uint32_t scratch = B * 4;
-        const uint32_t lds = scratch + 8 * (B / 32) * 4;
+        const uint32_t lds = scratch + prep_words(B / 32) * 4;
         hipLaunchKernelGGL(fg_prepare_kernel, dim3(nq), dim3(64), lds, nullptr, dq, ix->d_signs,
                            static_cast<int>(ix->dim), static_cast<int>(B), static_cast<int>(nq), drot, dqt, dl, ds,
                            scratch);
@@ -1129,8 +1131,9 @@ int fg_score_edges(fg_index *ix, const float *queries, uint32_t nq, const uint32
     S.use_ip = ix->metric == FG_METRIC_IP;
     S.n = n;
     S.query_off = B * 4;
-    S.plane_off = S.query_off + ((ix->dim + 3) & ~3u) * 4;
-    const uint32_t lds = S.plane_off + 8 * (B / 32) * 4;
+    S.prep_off = S.query_off + ((ix->dim + 3) & ~3u) * 4;
+    S.level_off = S.prep_off + prep_words(B / 32) * 4;
+    const uint32_t lds = S.level_off + B;
     float *dq = nullptr, *o1 = nullptr, *o2 = nullptr, *o3 = nullptr;
     uint32_t *t1 = nullptr, *t2 = nullptr, *t3 = nullptr;
     int rc = FG_OK;
