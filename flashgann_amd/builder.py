@@ -530,6 +530,11 @@ def codebook_from_graph(base, nbrs, signs: np.ndarray, use_ip: bool = False,
     if signs.shape[0] != lay.padded_dim:
         raise ValueError("signs must have padded_dim entries")
     b = lay.padded_dim
+    if entry is None:
+        entry = entry_point(x) if store_entry else MAX_INDEX
+    if x.is_cuda and n and 33 <= dim <= 2048 and 1 <= degree <= 1024:  # fg_encode_rows' range
+        rows = _encode_rows_gpu(x, nbrs, signs, lay, use_ip, verbose)
+        return Codebook(rows, np.asarray(signs, dtype=np.float32), int(entry), lay)
     p, pos, weights = _encode_setup(signs, x.device)
     rows = np.zeros((n, lay.row_offset), dtype=np.float32)
     code_bytes = rows[:, lay.code_offset : lay.factor_offset].view(np.uint8)
@@ -546,9 +551,49 @@ def codebook_from_graph(base, nbrs, signs: np.ndarray, use_ip: bool = False,
         ids[s:e] = np.where(nbh < 0, MAX_INDEX, nbh).astype(np.uint32)
         if verbose and (s // step) % 100 == 99:
             print(f"[builder] encoded {e}/{n} nodes", flush=True)
-    if entry is None:
-        entry = entry_point(x) if store_entry else MAX_INDEX
     return Codebook(rows, np.asarray(signs, dtype=np.float32), int(entry), lay)
+
+
+def _encode_rows_gpu(x: torch.Tensor, nbrs: torch.Tensor, signs: np.ndarray, lay: Layout, use_ip: bool,
+                     verbose: bool = False, stage_bytes: int = 1 << 23) -> np.ndarray:
+    """The rows of codebook_from_graph with the device's own encoding kernel
+    (fg_encode_rows): whole rows leave the device through two page-locked
+    staging blocks of at most `stage_bytes` (one row if that is more), and
+    while one is being filled the host copies the other into the result."""
+    from . import _lib
+    n, degree = nbrs.shape
+    x, nbrs = x.contiguous(), nbrs.contiguous()
+    if int(nbrs.max()) >= n:
+        raise IndexError(f"neighbour id out of range for {n} points")
+    sg = torch.as_tensor(np.ascontiguousarray(signs, dtype=np.float32), device=x.device)
+    rows = np.empty((n, lay.row_offset), dtype=np.float32)
+    out = torch.from_numpy(rows)
+    step = min(n, max(1, stage_bytes // lay.row_bytes))
+    metric = _lib.FG_METRIC_IP if use_ip else _lib.FG_METRIC_L2
+    pending = None
+    with torch.cuda.device(x.device):
+        stream = torch.cuda.current_stream()
+        dev = [torch.empty((step, lay.row_offset), dtype=torch.float32, device=x.device) for _ in range(2)]
+        host = [torch.empty((step, lay.row_offset), dtype=torch.float32, pin_memory=True) for _ in range(2)]
+        done = [torch.cuda.Event() for _ in range(2)]
+        for c, s in enumerate(range(0, n, step)):
+            m, k = min(step, n - s), c & 1
+            _lib.check(_lib.lib().fg_encode_rows(x.data_ptr(), n, lay.dim, degree, nbrs.data_ptr(), sg.data_ptr(),
+                                                 metric, s, m, dev[k].data_ptr(), stream.cuda_stream))
+            host[k][:m].copy_(dev[k][:m], non_blocking=True)
+            done[k].record(stream)
+            if pending is not None:
+                ps, pm, pk = pending
+                done[pk].synchronize()
+                out[ps:ps + pm].copy_(host[pk][:pm])
+            pending = (s, m, k)
+            if verbose and c % 100 == 99:
+                print(f"[builder] encoded {s + m}/{n} nodes", flush=True)
+        if pending is not None:
+            ps, pm, pk = pending
+            done[pk].synchronize()
+            out[ps:ps + pm].copy_(host[pk][:pm])
+    return rows
 
 
 def ground_truth(base, queries, k: int, device: str | torch.device = "cpu", use_ip: bool = False,

@@ -290,6 +290,164 @@ __global__ __launch_bounds__(256) void fg_dup_kernel(const float *rows, uint64_t
     }
 }
 
+// ------------------------------------------------------------ codebook encoding
+
+struct EncodeParams {
+    const float *base;         // n x dim
+    const int64_t *neighbors;  // n x degree, negative: empty slot
+    const float *signs;        // padded_dim
+    float *rows;               // row `first` of the codebook on
+    uint64_t n, first, row_offset, code_offset, factor_offset, neighbor_offset;
+    uint32_t dim, degree;
+    int use_ip;
+};
+
+// A double from lane l ^ M.
+template <int M>
+__device__ __forceinline__ double xshfl_d(double v) {
+    return __hiloint2double(xshfl(__double2hiint(v), M), xshfl(__double2loint(v), M));
+}
+template <int M, int K>
+__device__ __forceinline__ void rotate_lanes(double (&y)[K]) {
+    const bool upper = lane_in(lane_bit_mask(M));
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const double o = xshfl_d<M>(y[k]);
+        y[k] = upper ? o - y[k] : y[k] + o;
+    }
+}
+// Unnormalised Walsh-Hadamard transform of 64 K doubles, element lane + 64 k in
+// y[k] of each lane.
+template <int K>
+__device__ __forceinline__ void rotate_wave(double (&y)[K]) {
+    rotate_lanes<1>(y);
+    rotate_lanes<2>(y);
+    rotate_lanes<4>(y);
+    rotate_lanes<8>(y);
+    rotate_lanes<16>(y);
+    rotate_lanes<32>(y);
+#pragma unroll
+    for (int len = 1; len < K; len <<= 1)
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (!(k & len)) {
+                const double u = y[k], v = y[k | len];
+                y[k] = u + v;
+                y[k | len] = u - v;
+            }
+}
+__device__ __forceinline__ double wave_sum_d(double v) {
+    v += xshfl_d<32>(v);
+    v += xshfl_d<16>(v);
+    v += xshfl_d<8>(v);
+    v += xshfl_d<4>(v);
+    v += xshfl_d<2>(v);
+    return v + xshfl_d<1>(v);
+}
+
+// One codebook row per wave: the vector, then per edge the code bits and the
+// three factors (the definitions are the builder's: residual r = v - u, rotated
+// y = H diag(signs) r, bits y > 0, f = -2 |r|^2 / sum |y|), then the ids.  All
+// sums in fp64, as the builder's torch path.  That path multiplies by the
+// dense rotation (padded_dim^2 multiply-adds per edge) and makes some fifteen
+// passes over padded_dim doubles per edge; the fast transform in registers
+// leaves one read of each neighbour's vector and one write of the row, and
+// the row leaves the device whole: 50k points at d 128, degree 32 into a host
+// codebook 27.1 -> 2.9 ms (77 MB of rows through page-locked staging; the
+// copy, not this kernel, bounds it).  padded_dim = 64 K.
+template <int K>
+__global__ __launch_bounds__(64) void fg_encode_kernel(EncodeParams E) {
+    __shared__ double pc[64 * K];  // the rotated vector of the node
+    const int lane = lane_id();
+    const uint64_t node = E.first + blockIdx.x;
+    const float *u = E.base + node * E.dim;
+    float *row = E.rows + static_cast<uint64_t>(blockIdx.x) * E.row_offset;
+    float sg[K], cu[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const uint32_t i = static_cast<uint32_t>(lane) + 64u * k;
+        cu[k] = i < E.dim ? u[i] : 0.0f;
+        sg[k] = E.signs[i];
+        if (i < E.dim) row[i] = cu[k];
+    }
+    {
+        double y[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) y[k] = static_cast<double>(cu[k]) * static_cast<double>(sg[k]);
+        rotate_wave<K>(y);
+#pragma unroll
+        for (int k = 0; k < K; ++k) pc[lane + 64 * k] = y[k];
+    }
+    uint32_t *codes = reinterpret_cast<uint32_t *>(row + E.code_offset);
+    float *fac = row + E.factor_offset;
+    uint32_t *ids = reinterpret_cast<uint32_t *>(row + E.neighbor_offset);
+    const int64_t *nb = E.neighbors + node * E.degree;
+    for (uint32_t e0 = 0; e0 < E.degree; e0 += 64) {
+        const uint32_t ne = E.degree - e0 < 64u ? E.degree - e0 : 64u;
+        const int64_t mine = static_cast<uint32_t>(lane) < ne ? nb[e0 + lane] : -1;
+        const bool have = mine >= 0 && static_cast<uint64_t>(mine) < E.n;
+        const uint32_t id = have ? static_cast<uint32_t>(mine) : kMaxIndex;
+        // lane e keeps edge e0 + e's factors
+        float tx = FLT_MAX, fdq = 0.0f, fvq = 0.0f;
+        for (uint32_t e = 0; e < ne; ++e) {
+            const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(id), static_cast<int>(e)));
+            uint64_t bits[K];
+            if (v == kMaxIndex) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) bits[k] = 0ull;
+            } else {
+                const float *x = E.base + static_cast<uint64_t>(v) * E.dim;
+                double y[K], nr = 0.0, sabs = 0.0, spc = 0.0;
+                int ones = 0;
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const uint32_t i = static_cast<uint32_t>(lane) + 64u * k;
+                    const double r = i < E.dim ? static_cast<double>(x[i]) - static_cast<double>(cu[k]) : 0.0;
+                    nr += r * r;
+                    y[k] = r * static_cast<double>(sg[k]);
+                }
+                rotate_wave<K>(y);
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const uint64_t m = ballot(y[k] > 0.0);
+                    ones += __popcll(m);
+                    sabs += fabs(y[k]);
+                    const double p = pc[lane + 64 * k];
+                    spc += lane_in(m) ? p : -p;
+                    // dimension i of a 4-dimension chunk is bit 3 - i of its nibble
+                    bits[k] = (m & 0x1111111111111111ull) << 3 | (m & 0x2222222222222222ull) << 1 |
+                              (m & 0x4444444444444444ull) >> 1 | (m & 0x8888888888888888ull) >> 3;
+                }
+                nr = wave_sum_d(nr);
+                sabs = wave_sum_d(sabs);
+                spc = wave_sum_d(spc);
+                const bool zero = sabs <= 0.0;
+                const double f = zero ? 0.0 : (E.use_ip ? -nr : -2.0 * nr) / sabs;
+                const double t = zero || E.use_ip ? 0.0 : nr - f * spc;
+                if (static_cast<uint32_t>(lane) == e) {
+                    tx = static_cast<float>(t);
+                    fdq = static_cast<float>(f);
+                    fvq = static_cast<float>(f * static_cast<double>(2 * ones - 64 * K));
+                }
+            }
+            // the edge's 2 K code words, one per lane
+            uint32_t w = 0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                w = lane == 2 * k ? static_cast<uint32_t>(bits[k]) : w;
+                w = lane == 2 * k + 1 ? static_cast<uint32_t>(bits[k] >> 32) : w;
+            }
+            if (lane < 2 * K) codes[static_cast<uint64_t>(e0 + e) * (2 * K) + lane] = w;
+        }
+        if (static_cast<uint32_t>(lane) < ne) {
+            fac[e0 + lane] = tx;
+            fac[E.degree + e0 + lane] = fdq;
+            fac[2 * E.degree + e0 + lane] = fvq;
+            ids[e0 + lane] = id;
+        }
+    }
+}
+
 // ------------------------------------------------------------ test-hook kernels
 
 __global__ __launch_bounds__(64) void fg_prepare_kernel(const float *queries, const float *signs, int dim, int B,
@@ -1104,6 +1262,34 @@ int fg_search_noalloc(fg_index *ix, const float *queries, uint32_t nq, uint32_t 
     // (one launch: the two-launch search keeps its state in memory the index allocates)
     return search_host(ix, P, queries, nq, K, result_ids, counters, stats, reinterpret_cast<float *>(base),
                        reinterpret_cast<uint32_t *>(base + qb), reinterpret_cast<uint32_t *>(base + qb + rb), false);
+}
+
+int fg_encode_rows(const float *d_base, uint64_t npoints, uint32_t dim, uint32_t degree, const int64_t *d_neighbors,
+                   const float *d_signs, int metric, uint64_t first, uint64_t count, float *d_rows, void *stream) {
+    if (int rc = check_shape(dim, degree)) return rc;
+    if (metric != FG_METRIC_L2 && metric != FG_METRIC_IP) return fail(FG_EINVAL, "unknown metric");
+    if (npoints > 0xFFFFFFFFull || first > npoints || count > npoints - first || count > static_cast<uint64_t>(INT32_MAX))
+        return fail(FG_EINVAL, "rows to encode out of range");
+    if (count == 0) return FG_OK;
+    if (!d_base || !d_neighbors || !d_signs || !d_rows) return fail(FG_EINVAL, "NULL device buffer");
+    fg_index tmp;
+    tmp.dim = dim;
+    tmp.degree = degree;
+    compute_offsets(&tmp);
+    const EncodeParams E{d_base, d_neighbors, d_signs, d_rows, npoints, first, tmp.row_offset, tmp.code_offset,
+                         tmp.factor_offset, tmp.neighbor_offset, dim, degree, metric == FG_METRIC_IP};
+    const dim3 grid(static_cast<uint32_t>(count)), block(64);
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    switch (tmp.padded_dim / 64) {
+    case 1: hipLaunchKernelGGL(fg_encode_kernel<1>, grid, block, 0, st, E); break;
+    case 2: hipLaunchKernelGGL(fg_encode_kernel<2>, grid, block, 0, st, E); break;
+    case 4: hipLaunchKernelGGL(fg_encode_kernel<4>, grid, block, 0, st, E); break;
+    case 8: hipLaunchKernelGGL(fg_encode_kernel<8>, grid, block, 0, st, E); break;
+    case 16: hipLaunchKernelGGL(fg_encode_kernel<16>, grid, block, 0, st, E); break;
+    default: hipLaunchKernelGGL(fg_encode_kernel<32>, grid, block, 0, st, E); break;
+    }
+    FG_HIP(hipGetLastError(), "encode kernel launch");
+    return FG_OK;
 }
 
 int fg_query_prepare(fg_index *ix, const float *queries, uint32_t nq, float *rotated, uint8_t *quantized,

@@ -204,6 +204,17 @@ int fg_search_launches(fg_index *index, uint32_t nq, uint32_t K, uint32_t beam);
 #define FG_GEOMETRY_GENERAL 1
 int fg_search_geometry(const fg_index *index);
 
+/* Encodes `count` codebook rows from row `first` on the device (the builder's
+ * last step; the reference consumes a prebuilt codebook and has no
+ * counterpart): per node its vector, each edge's 1-bit code and three factors,
+ * and its neighbour ids, in the layout of fg_index_info.  d_base: npoints x dim
+ * float32; d_neighbors: npoints x degree int64, negative for an empty slot
+ * (an id past the last point is taken as one); d_signs: padded_dim float32;
+ * d_rows: count rows.  Enqueued on `stream`, no synchronisation, no
+ * allocation. */
+int fg_encode_rows(const float *d_base, uint64_t npoints, uint32_t dim, uint32_t degree, const int64_t *d_neighbors,
+                   const float *d_signs, int metric, uint64_t first, uint64_t count, float *d_rows, void *stream);
+
 /* Query preparation only (utils.cuh:840-939): rotated query (padded_dim
  * float32), quantized levels (padded_dim uint8), and {low, high, width} plus
  * sum_q, for nq host queries.  Test hook for the preparation stage. */

@@ -87,3 +87,35 @@ def test_search_on_partitioned_gpu_build_1536(gpu_available):
     gt = builder.ground_truth(base, q, 100, device="cuda")
     from flashgann_amd.metrics import compute_recall
     assert compute_recall(ids, gt, 100) > 0.9
+
+
+@pytest.mark.parametrize("dim,degree,use_ip", [(33, 1, False), (64, 3, True), (65, 64, False), (100, 65, True),
+                                               (128, 130, False), (200, 24, True), (512, 31, False), (960, 32, True),
+                                               (1536, 16, False), (2048, 8, True)])
+def test_gpu_encode_kernel_equals_cpu_encoding(gpu_available, dim, degree, use_ip):
+    """fg_encode_rows (every register count of its transform, degrees around
+    its 64-edge blocks, a last staging block that is not full) against the
+    torch path on the CPU.  Integer data with empty slots, a node linked to
+    itself and a repeated point: all sums are whole numbers below 2^53 in
+    both, and the one division rounds once, so the rows are the same bytes."""
+    import torch
+    from flashgann_amd import builder, datasets
+    from flashgann_amd.codebook import padded_dim_for
+    n = 301
+    rng = np.random.default_rng(dim + degree)
+    base = rng.integers(-40, 200, size=(n, dim)).astype(np.float32)
+    base[7] = base[5]
+    nbrs = rng.integers(0, n, size=(n, degree))
+    nbrs[rng.random((n, degree)) < 0.1] = -1
+    nbrs[3, 0] = 3
+    nbrs[5, -1] = 7
+    signs = datasets.signs_for(padded_dim_for(dim))
+    a = builder.codebook_from_graph(base, nbrs, signs, use_ip=use_ip, device="cpu", entry=0)
+    b = builder.codebook_from_graph(base, nbrs, signs, use_ip=use_ip, device="cuda", entry=0)
+    assert np.array_equal(a.rows.view(np.uint32), b.rows.view(np.uint32))
+    x, nb = torch.as_tensor(base).cuda(), torch.as_tensor(nbrs).cuda()
+    c = builder._encode_rows_gpu(x, nb, signs, a.layout, use_ip, stage_bytes=7 * a.layout.row_bytes)
+    assert np.array_equal(a.rows.view(np.uint32), c.view(np.uint32))
+    nb[0, 0] = n
+    with pytest.raises(IndexError):
+        builder._encode_rows_gpu(x, nb, signs, a.layout, use_ip)
