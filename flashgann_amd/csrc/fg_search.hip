@@ -847,6 +847,9 @@ uint64_t slice_buffer_words(const SearchParams &P, uint64_t *states_out, uint64_
     return words;
 }
 
+// fg_search_stream's largest launch of several batches.
+constexpr uint32_t kStreamQueries = 16384;
+
 bool slice_wanted(const SearchParams &P) {
     if (P.nq < 1 || P.max_iter <= kSliceStop) return false;
     return slice_buffer_words(P, nullptr, nullptr) * 4u <= kSliceMaxBytes;
@@ -1129,6 +1132,21 @@ int fg_search_stream(fg_index *ix, const float *d_queries, uint32_t nq, uint32_t
     if (int rc = make_params(ix, batch < nq ? batch : nq, K, beam, P)) return rc;
     if (nq == 0) return FG_OK;
     hipStream_t caller = reinterpret_cast<hipStream_t>(stream);
+    // Consecutive batches of up to kStreamQueries queries share a launch: a
+    // small batch leaves most of the device idle and ends in a tail of its
+    // longest searches, and one launch of them all pays both once.  8 batches
+    // of 1,000 queries (d 128, beam 128) on two streams: 1.002 -> 0.515 ms.
+    // The bound keeps a launch's two-launch state small (40 MB at beam 256)
+    // and its order step in one workgroup.
+    const uint32_t per = batch < kStreamQueries ? batch * (kStreamQueries / batch) : batch;
+    if (nq <= per) {
+        P.nq = static_cast<int>(nq);
+        P.queries = d_queries;
+        P.results = d_results;
+        P.counters = nullptr;
+        P.phase = nullptr;
+        return launch(ix, P, caller, true);
+    }
     while (ix->serve_count < static_cast<int>(nstreams)) {
         const int i = ix->serve_count;
         FG_HIP(hipStreamCreateWithFlags(&ix->serve[i], hipStreamNonBlocking), "serving stream");
@@ -1139,14 +1157,14 @@ int fg_search_stream(fg_index *ix, const float *d_queries, uint32_t nq, uint32_t
         ix->serve_count = i + 1;
     }
     if (!ix->serve_start) FG_HIP(hipEventCreateWithFlags(&ix->serve_start, hipEventDisableTiming), "serving event");
-    // every batch runs after the work already queued on the caller's stream
+    // every launch runs after the work already queued on the caller's stream
     FG_HIP(hipEventRecord(ix->serve_start, caller), "event record");
-    const uint32_t nbatch = (nq + batch - 1) / batch;
-    const uint32_t used = nbatch < nstreams ? nbatch : nstreams;
+    const uint32_t nlaunch = (nq - 1) / per + 1;
+    const uint32_t used = nlaunch < nstreams ? nlaunch : nstreams;
     for (uint32_t i = 0; i < used; ++i) FG_HIP(hipStreamWaitEvent(ix->serve[i], ix->serve_start, 0), "stream wait");
-    for (uint32_t b = 0; b < nbatch; ++b) {
-        const uint64_t q0 = static_cast<uint64_t>(b) * batch;
-        const uint32_t n = static_cast<uint32_t>(nq - q0 < batch ? nq - q0 : batch);
+    for (uint32_t b = 0; b < nlaunch; ++b) {
+        const uint64_t q0 = static_cast<uint64_t>(b) * per;
+        const uint32_t n = static_cast<uint32_t>(nq - q0 < per ? nq - q0 : per);
         SearchParams Pb = P;
         Pb.nq = static_cast<int>(n);
         Pb.queries = d_queries + q0 * ix->dim;
@@ -1155,7 +1173,7 @@ int fg_search_stream(fg_index *ix, const float *d_queries, uint32_t nq, uint32_t
         Pb.phase = nullptr;
         if (int rc = launch(ix, Pb, ix->serve[b % nstreams], false)) return rc;
     }
-    // and the caller's later work runs after every batch
+    // and the caller's later work runs after every launch
     for (uint32_t i = 0; i < used; ++i) {
         FG_HIP(hipEventRecord(ix->serve_done[i], ix->serve[i]), "event record");
         FG_HIP(hipStreamWaitEvent(caller, ix->serve_done[i], 0), "stream wait");

@@ -135,14 +135,17 @@ int fg_search_device(fg_index *index, const float *d_queries, uint32_t nq, uint3
 /* Serving form of fg_search_device for a stream of query batches (the
  * reference has no counterpart: its gpu_search_adaptive.cu:99-103 launches
  * one kernel per call and synchronises).  The nq device-resident queries are
- * searched as consecutive batches of `batch` queries, batch b on internal
- * stream b % nstreams (1 <= nstreams <= 8, created on first use and owned by
- * the index), so one batch's last, partly filled wave slots overlap the next
- * batch's start.  Results land in query order in d_results (nq x K); each
- * query's ids are those fg_search_device returns.  All batches run after the
- * work already queued on `stream` and that stream's later work waits for
- * all of them; the call returns without synchronising.  Calls on one index
- * share its internal streams: issue them from one host thread. */
+ * searched in batches of `batch`: consecutive batches of together up to
+ * 16,384 queries share a launch, and when there are several launches they go
+ * round `nstreams` internal streams (1 <= nstreams <= 8, created on first use
+ * and owned by the index), so one launch's last, partly filled wave slots
+ * overlap the next one's start.  A call that needs one launch makes it on
+ * `stream`, as fg_search_device would.  Results land in query order in
+ * d_results (nq x K); each query's ids are those fg_search_device returns.
+ * All batches run after the work already queued on `stream` and that stream's
+ * later work waits for all of them; the call returns without synchronising.
+ * Calls on one index share its internal streams: issue them from one host
+ * thread. */
 int fg_search_stream(fg_index *index, const float *d_queries, uint32_t nq, uint32_t K, uint32_t beam,
                      uint32_t *d_results, uint32_t batch, uint32_t nstreams, void *stream);
 
@@ -185,8 +188,9 @@ int fg_search_waves(fg_index *index, uint32_t nq, uint32_t K, uint32_t beam);
  * Results are identical either way; FLASHGANN_SLICE=0/1 in the environment
  * forces one launch / two wherever the form allows.  Device searches on one index that
  * overlap on different streams run one after another when they take two
- * launches.  fg_search_stream, fg_search_noalloc and a device search on a
- * stream that is being captured into a graph always make one.
+ * launches.  fg_search_noalloc, the several launches of one fg_search_stream
+ * call and a device search on a stream that is being captured into a graph
+ * are never split in two.
  * Negative FG_E* on invalid arguments.  No counterpart in the reference (one
  * launch per call, gpu_search_adaptive.cu:99-103). */
 int fg_search_launches(fg_index *index, uint32_t nq, uint32_t K, uint32_t beam);
