@@ -792,8 +792,8 @@ __device__ __forceinline__ void raw_span(const uint32_t *const (&code)[NB], cons
     }
 }
 
-// raw of NB neighbour codes per lane of W words each (W a power of two >= 8:
-// padded dimension >= 256), loaded up to NWD words at a time with 16-byte
+// raw of NB neighbour codes per lane of W words each (W a power of two >= 16:
+// padded dimension >= 512), loaded up to NWD words at a time with 16-byte
 // loads when the row layout keeps codes 16-byte aligned.  Every lane of the
 // wave comes here (the matrix unit takes all lanes' operands).  The codes of
 // lanes outside `want` are not read: such a lane feeds whatever its registers
@@ -813,10 +813,8 @@ __device__ __forceinline__ void raw_words(const uint32_t *const (&code)[NB], con
     const LevelRows lr = level_rows(static_cast<uint32_t>(W));
     if (W >= 32) {
         for (int w0 = 0; w0 < W; w0 += 32) raw_span<NB, 32>(code, want, prep, lr, W, w0, vec_ok, any_wrap, acc, wraps);
-    } else if (W == 16) {
-        raw_span<NB, 16>(code, want, prep, lr, W, 0, vec_ok, any_wrap, acc, wraps);
     } else {
-        raw_span<NB, 8>(code, want, prep, lr, W, 0, vec_ok, any_wrap, acc, wraps);
+        raw_span<NB, 16>(code, want, prep, lr, W, 0, vec_ok, any_wrap, acc, wraps);
     }
 #pragma unroll
     for (int b = 0; b < NB; ++b) raw[b] = raw_value(acc[b]) - static_cast<float>(256u * wraps[b]);
@@ -1446,10 +1444,13 @@ __device__ __forceinline__ void controller_step(Controller &c, uint32_t beam0, f
 // the row layout keeps the code block 16-byte aligned).
 template <int WT>
 __device__ __forceinline__ void load_code(const uint32_t *__restrict__ code, bool vec_ok, uint32_t (&c)[WT]) {
-    if constexpr (WT == 4) {
+    if constexpr (WT % 4 == 0) {
         if (vec_ok) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(code);
-            c[0] = v.x; c[1] = v.y; c[2] = v.z; c[3] = v.w;
+#pragma unroll
+            for (int j = 0; j < WT / 4; ++j) {
+                const uint4 v = reinterpret_cast<const uint4 *>(code)[j];
+                c[4 * j] = v.x; c[4 * j + 1] = v.y; c[4 * j + 2] = v.z; c[4 * j + 3] = v.w;
+            }
             return;
         }
     }
@@ -1599,8 +1600,13 @@ __device__ __forceinline__ void exact_batch_range(const SearchParams &P, const G
     const int h = lane >> 5, nl = lane & 31;
     const bool ip = sflag(static_cast<uint32_t>(P.use_ip));
     if constexpr (DPL > 0) {
+        // (8 floats per lane and row: eight children a pass, for the registers)
         int e0 = lo;
-        for (; n - e0 > 8; e0 += 16) exact_pass<8, DPL>(P, g, e0, n, slot_list, cd, ci, qr, ip);
+        if constexpr (DPL > 4) {
+            for (; n - e0 > 8; e0 += 8) exact_pass<4, DPL>(P, g, e0, n, slot_list, cd, ci, qr, ip);
+        } else {
+            for (; n - e0 > 8; e0 += 16) exact_pass<8, DPL>(P, g, e0, n, slot_list, cd, ci, qr, ip);
+        }
         const int rem = n - e0;
         if (rem > 4) exact_pass<4, DPL>(P, g, e0, n, slot_list, cd, ci, qr, ip);
         else if (rem > 2) exact_pass<2, DPL>(P, g, e0, n, slot_list, cd, ci, qr, ip);
@@ -1764,7 +1770,7 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
 // exact distances; `lead_sync` orders the lead wave's own LDS accesses and
 // the workgroup barriers mark the meeting points.
 template <int WT, int DPL, int DIM_T, int DEG_T, bool COUNT, bool PROF, bool BIG, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? 3 : 5))) void fg_search_kernel(SearchParams P) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? 3 : WT > 4 ? 4 : 5))) void fg_search_kernel(SearchParams P) {
     static_assert(NW == 1 || NW == 2, "team form: two waves");
     extern __shared__ __align__(16) unsigned char smem[];
     int qid = blockIdx.x;
@@ -2673,9 +2679,9 @@ void launch_geo(const SearchParams &P, hipStream_t stream, bool count, bool prof
 }
 
 // Launch functions of the shape classes, one translation unit each
-// (fg_shapes.hip with FG_SHAPE = 0 .. 6): d 128 / degree 32, d 96 / degree
+// (fg_shapes.hip with FG_SHAPE = 0 .. 7): d 128 / degree 32, d 96 / degree
 // 32, d 96 / degree 16 (compile-time geometry), then the runtime-geometry
-// kernels for padded dimension 64, 128 with d <= 96, 128, and >= 256.
+// kernels for padded dimension 64, 128 with d <= 96, 128, >= 512, and 256.
 using LaunchShape = void (*)(const SearchParams &, hipStream_t, bool count, bool prof, int *waves_only,
                              bool one_wave, long long *resident);
 void launch_shape0(const SearchParams &, hipStream_t, bool, bool, int *, bool, long long *);
@@ -2685,5 +2691,6 @@ void launch_shape3(const SearchParams &, hipStream_t, bool, bool, int *, bool, l
 void launch_shape4(const SearchParams &, hipStream_t, bool, bool, int *, bool, long long *);
 void launch_shape5(const SearchParams &, hipStream_t, bool, bool, int *, bool, long long *);
 void launch_shape6(const SearchParams &, hipStream_t, bool, bool, int *, bool, long long *);
+void launch_shape7(const SearchParams &, hipStream_t, bool, bool, int *, bool, long long *);
 
 }  // namespace fgk

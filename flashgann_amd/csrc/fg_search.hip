@@ -530,6 +530,10 @@ __global__ __launch_bounds__(64) void fg_score_kernel(ScoreParams S) {
         uint32_t c[1][2];
         load_code<2>(code, vec_ok, c[0]);
         raw_batch<1, 2>(c, prep, any_wrap, r);
+    } else if (W == 8) {
+        uint32_t c[1][8];
+        load_code<8>(code, vec_ok, c[0]);
+        raw_batch<1, 8>(c, prep, any_wrap, r);
     } else {
         const uint32_t *const cp[1] = {code};
         const uint64_t all[1] = {~0ull};
@@ -813,6 +817,14 @@ int launch_t(const SearchParams &P, hipStream_t stream, int *waves_only = nullpt
         launch_shape4(P, stream, count, PROF, waves_only, one_wave, resident);
     } else if (W == 4) {
         launch_shape5(P, stream, count, PROF, waves_only, one_wave, resident);
+    } else if (W == 8) {
+        // padded dimension 256: 8 code words and 8 floats a lane are few
+        // enough for registers, so codes and factors come with the ids (one
+        // round trip instead of two) and a pass loads a row's own dimensions
+        // (the wider kernels' batch of 16 steps of 32 loads past them):
+        // 777 queries at d 200, degree 32, beam 300, inner product 0.604 ->
+        // 0.497 ms
+        launch_shape7(P, stream, count, PROF, waves_only, one_wave, resident);
     } else {
         launch_shape6(P, stream, count, PROF, waves_only, one_wave, resident);
     }

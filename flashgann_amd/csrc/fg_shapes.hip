@@ -1,11 +1,11 @@
 // fg_shapes.hip -- one shape class of the search kernel per object file:
-// compiled once for each FG_SHAPE = 0 .. 6 (see the Makefile), so the
+// compiled once for each FG_SHAPE = 0 .. 7 (see the Makefile), so the
 // classes' kernels compile in parallel.  fg_search.hip's launch_t picks the
-// class (fg_kernel.hpp declares the seven launch functions).
+// class (fg_kernel.hpp declares the eight launch functions).
 #include "fg_kernel.hpp"
 
 #ifndef FG_SHAPE
-#error "compile with -DFG_SHAPE=0..6"
+#error "compile with -DFG_SHAPE=0..7"
 #endif
 
 namespace fgk {
@@ -28,9 +28,11 @@ void launch_shape4(FG_SHAPE_ARGS) { launch_geo<4, 3, 0, 0>(FG_SHAPE_CALL); }  //
 #elif FG_SHAPE == 5
 void launch_shape5(FG_SHAPE_ARGS) { launch_geo<4, 4, 0, 0>(FG_SHAPE_CALL); }  // padded 128
 #elif FG_SHAPE == 6
-void launch_shape6(FG_SHAPE_ARGS) { launch_geo<0, 0, 0, 0>(FG_SHAPE_CALL); }  // padded dim >= 256
+void launch_shape6(FG_SHAPE_ARGS) { launch_geo<0, 0, 0, 0>(FG_SHAPE_CALL); }  // padded dim >= 512
+#elif FG_SHAPE == 7
+void launch_shape7(FG_SHAPE_ARGS) { launch_geo<8, 8, 0, 0>(FG_SHAPE_CALL); }  // padded dim 256
 #else
-#error "FG_SHAPE must be 0..6"
+#error "FG_SHAPE must be 0..7"
 #endif
 
 }  // namespace fgk
