@@ -19,6 +19,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/flashgann.h"
@@ -1025,7 +1026,89 @@ __device__ __forceinline__ void sort32(float &key, uint32_t &val) {
     val = v[0];
 }
 
+// Places of SPAN (8, 16 or 32) keys in their sorted order, counted instead of
+// sorted: a key's place is the number of keys below it, found by comparing it
+// with the keys of lanes l ^ 1 .. l ^ (SPAN - 1).  Both 32-lane halves hold the
+// same keys, so each does half of the distances and one addition joins the
+// counts: 8 independent compares for 16 keys, where the network is 10
+// dependent exchanges of about seven instructions each.  `empty` marks the
+// (FLT_MAX, MAX_INDEX) pairs, which go last in lane order; every other key lies
+// in (-FLT_MAX, FLT_MAX).  Lanes nl >= SPAN are empty and keep their place.
+//
+// Returns whether the order is the network's: the sorted order of distinct
+// keys is unique, but equal keys end where the network moves them.  Of the
+// SPAN (SPAN - 1) / 2 pairs each has one lane that sees the other's key below
+// its own, unless the two are equal, as any two empties are.
+template <int SPAN>
+__device__ __forceinline__ bool sort_places(float key, bool empty, int &place) {
+    const int nl = lane_id() & 31;
+    const auto dpp = [](float v, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    constexpr std::integral_constant<int, 0x141> kHalfMirror{};  // l ^ 7
+    constexpr std::integral_constant<int, 0x140> kRowMirror{};   // l ^ 15
+    constexpr std::integral_constant<int, 0x128> kRowRor8{};     // l ^ 8
+    constexpr std::integral_constant<int, 0xB1> kXor1{};
+    constexpr std::integral_constant<int, 0x4E> kXor2{};
+    constexpr std::integral_constant<int, 0x1B> kXor3{};
+    // the upper half starts from the distance that its share lies around
+    const float far = SPAN == 32 ? xshfl(key, 16) : SPAN == 16 ? dpp(key, kRowMirror) : dpp(key, kHalfMirror);
+    const float c = lane_in(0xFFFFFFFF00000000ull) ? far : key;
+    constexpr int NB = SPAN / 8;
+    float base[NB];
+    base[0] = c;
+    if constexpr (NB > 1) base[1] = dpp(c, kHalfMirror);
+    if constexpr (NB > 2) {
+        base[2] = dpp(c, kRowMirror);
+        base[3] = dpp(c, kRowRor8);
+    }
+    constexpr uint32_t kLanes = SPAN == 32 ? 0xFFFFFFFFu : (1u << (SPAN & 31)) - 1u;
+    int below = 0, seen = 0;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const float o[4] = {base[b], dpp(base[b], kXor1), dpp(base[b], kXor2), dpp(base[b], kXor3)};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint64_t m = ballot(o[q] < key);
+            seen += __popcll(m);  // (the empty lanes past SPAN see none)
+            below += lane_in(m) ? 1 : 0;
+        }
+    }
+    below = add32i(below);
+    const uint32_t em = static_cast<uint32_t>(ballot(empty)) & kLanes;
+    const int e = __popc(em);
+    const int last = SPAN - e + static_cast<int>(__builtin_amdgcn_mbcnt_lo(em, 0));
+    place = empty ? last : below;
+    place = nl < SPAN ? place : nl;
+    return seen == SPAN * (SPAN - 1) / 2 - e * (e - 1) / 2;
+}
+
 __device__ __forceinline__ float pair_key(uint2 e) { return __uint_as_float(e.x); }
+
+// Sorts 32 pairs (position lane & 31, both halves the same) into ms[0 .. 31] in
+// the order of warp_sort<1> (utils.cuh:409-414).  `span`: pairs at or past it
+// are (FLT_MAX, MAX_INDEX).  `clean`: every key is in (-FLT_MAX, FLT_MAX) or
+// belongs to such a pair.
+__device__ __forceinline__ void sort_to(uint2 *ms, float key, uint32_t val, int span, bool clean) {
+    const int lane = lane_id();
+    if (clean) {
+        const bool empty = val == kMaxIndex;
+        int place;
+        bool distinct;
+        if (span <= 8) distinct = sort_places<8>(key, empty, place);
+        else if (span <= 16) distinct = sort_places<16>(key, empty, place);
+        else distinct = sort_places<32>(key, empty, place);
+        if (distinct) {
+            if (lane < 32) ms[place] = make_uint2(__float_as_uint(key), val);
+            return;
+        }
+    }
+    // (a network short of 32 needs every key of the span at most FLT_MAX)
+    if (clean && span <= 8) sort32<8>(key, val);
+    else if (clean && span <= 16) sort32<16>(key, val);
+    else sort32(key, val);
+    if (lane < 32) ms[lane] = make_uint2(__float_as_uint(key), val);
+}
 
 // Small merge, pbeam <= 128: topk_small_by_bitonic_sort<1, pbeam/32>
 // (utils.cuh:490-586).  Beam position p takes sorted candidate pbeam-1-p when
@@ -1223,10 +1306,9 @@ __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, con
 
 // Beam merge (utils.cuh:1369-1399 dispatch for a <= 32-entry buffer): the
 // candidates (slot s: distance cd[2 s], id ci[2 s], the pairs of `ms`) are
-// read into registers, sorted (warp_sort<1>), written back to `ms` in sorted
-// order, and merged into the beam in place.  `span`: slots at or past it hold (FLT_MAX, MAX_INDEX), so a
-// candidate buffer filled only in its first 8 or 16 slots is sorted with the
-// stages that reach that block size (sort32<TOP>).  `fast_ok` stays true while
+// read into registers, written back to `ms` in sorted order (sort_to), and
+// merged into the beam in place.  `span`: slots at or past it hold (FLT_MAX,
+// MAX_INDEX).  `fast_ok` stays true while
 // every pair merged into this beam has a key in (-FLT_MAX, FLT_MAX) or is the
 // empty (FLT_MAX, MAX_INDEX) pair (merge_path's condition for its split
 // search).
@@ -1236,17 +1318,14 @@ __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uin
                                            const uint32_t *ci, int span, bool &fast_ok, int &lb_out) {
     const int lane = lane_id_opaque();
     lb_out = 0;
-    const int nl = lane & 31, h = lane >> 5;
+    const int nl = lane & 31;
     const int cbs = P.cbs, pbeam = P.pbeam;
-    float ck = nl < cbs ? cd[2 * nl] : FLT_MAX;
-    uint32_t cv = nl < cbs ? ci[2 * nl] : kMaxIndex;
-    fast_ok = fast_ok && !any_lane(!((ck > -FLT_MAX && ck < FLT_MAX) || (ck == FLT_MAX && cv == kMaxIndex)));
-    // every key of the span at most FLT_MAX (never inf or NaN)
-    const bool short_ok = !any_lane(nl < span && !(ck <= FLT_MAX));
-    if (short_ok && span <= 8) sort32<8>(ck, cv);
-    else if (short_ok && span <= 16) sort32<16>(ck, cv);
-    else sort32(ck, cv);
-    if (h == 0) ms[nl] = make_uint2(__float_as_uint(ck), cv);
+    const float ck = nl < cbs ? cd[2 * nl] : FLT_MAX;
+    const uint32_t cv = nl < cbs ? ci[2 * nl] : kMaxIndex;
+    const bool clean =
+        !any_lane(!(((ck > -FLT_MAX) & (ck < FLT_MAX) & (cv != kMaxIndex)) | ((ck == FLT_MAX) & (cv == kMaxIndex))));
+    fast_ok = fast_ok && clean;
+    sort_to(ms, ck, cv, span, clean);
     lead_sync<NW>();
     if constexpr (!BIG) {
         if (pbeam == 128) {
@@ -1254,7 +1333,7 @@ __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uin
         } else if (pbeam == 64) {
             small_merge<1, false>(pbeam, bp, ms, lane, true);
         } else if (pbeam == 32) {
-            small_merge<1, true>(pbeam, bp, ms, nl, h == 0);
+            small_merge<1, true>(pbeam, bp, ms, nl, lane < 32);
         } else {
             merge_path<1, NW>(P, bp, ms, fast_ok, 0);  // one segment per lane: nothing to save
         }
@@ -2173,11 +2252,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                         near = __popc(half_bits(ballot(child != kMaxIndex && isfinite(dist) && dist <= kth), 0));
                     const int eff = keep_count_for_expander(static_cast<uint32_t>(cwc), 1, ctl.rho, kth_valid, near);
                     // dispatch_candidate_bitonic_sort over the cbs-entry buffer (padding beyond it)
-                    float sk = nl < cbs ? dist : FLT_MAX;
-                    uint32_t sv = nl < cbs ? child : kMaxIndex;
-                    sort32(sk, sv);
-                    dist = sk;
-                    child = sv;
+                    const float sk = nl < cbs ? dist : FLT_MAX;
+                    const uint32_t sv = nl < cbs ? child : kMaxIndex;
+                    // (the runtime geometry of padded dimension 64 and 128 has no
+                    // registers left for the counted sort here as well)
+                    const bool clean = (kFixedGeo || WT == 0 || WT > 4) &&
+                                       !any_lane(!(((sk > -FLT_MAX) & (sk < FLT_MAX) & (sv != kMaxIndex)) |
+                                                   ((sk == FLT_MAX) & (sv == kMaxIndex))));
+                    sort_to(ms, sk, sv, 32, clean);
+                    lead_sync<NW>();
+                    const uint2 sorted = ms[nl];
+                    dist = pair_key(sorted);
+                    child = sorted.y;
                     if (nl >= eff) {
                         child = kMaxIndex;
                         dist = FLT_MAX;
