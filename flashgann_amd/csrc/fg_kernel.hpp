@@ -127,8 +127,7 @@ __host__ __device__ inline uint32_t visited_buckets_roomy(uint32_t beam, uint32_
 }
 
 struct LdsLayout {
-    uint32_t hash_off, beam_off, msort_off, prep_off, scratch_off, prof_off, total, total_prof, team_off,
-        total_team;
+    uint32_t hash_off, beam_off, msort_off, prep_off, scratch_off, total, total_team;
 };
 
 // Candidate buffer and sorted-candidate staging of the beam merge, one array
@@ -144,25 +143,28 @@ constexpr uint32_t kMsortPairs = 37;
 // slots are written to pbeam + 2).
 constexpr uint32_t kBeamPad = 4;
 
-// A team launch runs each query on two waves: the lead wave runs the search,
+// A team launch runs each query on two waves: the lead wave runs the search;
 // the helper takes half of every stage-II round (visited tests, estimates
-// and keep decisions of its tasks) and half of every exact-distance batch.
-// They meet at workgroup barriers and exchange through this LDS block.
+// and keep decisions of its tasks), half of every exact-distance batch, half
+// of every visited-table rebuild and, at beams over 256, half of the merge's
+// segments.  They meet at workgroup barriers and exchange through this LDS
+// block.
 struct TeamBlock {
     // per iteration, from the lead wave: stop flag, theta, rho, K-th cutoff,
     // number of expanders; then the exact batch's size and list kind
-    uint32_t stop, theta, nexp, kth_bits, rho_bits, ex_n, ex_alist, pad0;
+    uint32_t stop, theta, nexp, kth_bits, rho_bits, ex_n, ex_alist;
     // per query (written once): the quantised query's constants
-    uint32_t sum_q, qwidth_bits, qlow_bits, any_wrap, pad2;
+    uint32_t sum_q, qwidth_bits, qlow_bits, any_wrap;
     // the helper's work counters (counting build)
-    uint32_t c_ids, c_est, pad1;
-    // the helper's stage-II results: kept-lane masks and child ids of its
-    // sub-rounds
-    uint64_t klm[2];
-    uint32_t cid[2][64];
+    uint32_t c_ids, c_est;
+    // the helper's stage-II results: the kept children of its sub-rounds, in
+    // (task, lane) order (at most 4 per task at theta = 8)
+    uint32_t n_list;
+    uint32_t list[32];
 };
-constexpr uint32_t kTeamBytes = 640;
+constexpr uint32_t kTeamBytes = 192;
 static_assert(sizeof(TeamBlock) <= kTeamBytes, "team block");
+constexpr uint32_t kProfBytes = 16u * 8u;
 
 // The lead wave's way out of the search loop in the team form: it tells the
 // helper to stop at their meeting point (the helper then leaves too).
@@ -204,12 +206,9 @@ __host__ __device__ constexpr LdsLayout lds_layout(uint32_t dim, uint32_t padded
     off += buckets * 16u;
     if (off < L.beam_off + padded_dim * 4u) off = L.beam_off + padded_dim * 4u;
     L.total = (off + 15u) & ~15u;
-    // phase timers of the profiling build only, past the end of the rest
-    L.prof_off = L.total;
-    L.total_prof = L.total + 16u * 8u;
-    // a team launch's exchange block, past the phase timers
-    L.team_off = L.total_prof;
-    L.total_team = L.total_prof + kTeamBytes;
+    // a team launch's exchange block, past the rest; the profiling build's
+    // phase timers (kProfBytes) come after either
+    L.total_team = L.total + kTeamBytes;
     return L;
 }
 
@@ -226,7 +225,10 @@ __host__ __device__ inline uint32_t visited_buckets(uint32_t dim, uint32_t padde
                                                     uint32_t degree) {
     const uint32_t lo = visited_buckets_min(beam, degree);
     const uint32_t total = lds_layout(dim, padded_dim, pbeam, lo).total;
-    const uint32_t cap = (total + kLdsGranule - 1u) / kLdsGranule * kLdsGranule;
+    uint32_t cap = (total + kLdsGranule - 1u) / kLdsGranule * kLdsGranule;
+    // (room for the team form's block where it fits in the same granules: at
+    // beam 1024 the team form then holds as many queries as the one-wave form)
+    if (total + kTeamBytes <= cap) cap -= kTeamBytes;
     uint32_t b = visited_buckets_roomy(beam, degree);
     while (b > lo && lds_layout(dim, padded_dim, pbeam, b).total > cap) --b;
     return b;
@@ -1163,11 +1165,16 @@ __device__ __forceinline__ void small_merge(int pbeam, uint2 *bp, const uint2 *m
 // outside (-FLT_MAX, FLT_MAX) has been merged into this beam), and every
 // split of such a tie gives the same output.  Any other equal pair sends the
 // whole wave through the reference's bisection, replayed step by step.
-template <int SPL, int NW = 1>
-__device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, const uint2 *ms, bool fast_ok,
-                                           int tbase) {
+//
+// SPLIT: both waves of a team take part, each with its own range of segments
+// (tbase, active); the waves meet between the reads and the writes.  The
+// second wave's range starts one segment early, for that segment's right
+// boundary alone (`shadow`: it is not written).
+template <int SPL, int NW = 1, bool SPLIT = false>
+__device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, const uint2 *ms, bool fast_ok, int tbase,
+                                           int active, bool shadow = false) {
     const int lane = lane_id_opaque();
-    const int cbs = P.cbs, pbeam = P.pbeam, active = P.seg_active;
+    const int cbs = P.cbs, pbeam = P.pbeam;
     // step k of lane l: segment tbase + 64 k + l (consecutive lanes, and so
     // nearby LDS addresses, in every step)
     int tk[SPL], dl[SPL], dr[SPL], rl[SPL], rr[SPL];
@@ -1270,6 +1277,8 @@ __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, con
         const int tb = act ? rl[k] : 0;
         const int cb = act ? dl[k] - rl[k] : 0;
         nsl[k] = act ? dr[k] - dl[k] : 0;
+        if constexpr (SPLIT)
+            if (k == 0 && shadow && lane == 0) nsl[k] = 0;
         // The bisection resolves equal keys at each boundary on its own, so
         // two boundaries can disagree (seen at the first merge, where every
         // entry is the empty pair): more than nsl beam entries, or fewer
@@ -1297,7 +1306,8 @@ __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, con
             }
     }
     // every lane has read its inputs before any output overwrites them
-    lead_sync<NW>();
+    if constexpr (SPLIT) __syncthreads();
+    else lead_sync<NW>();
 #pragma unroll
     for (int k = 0; k < SPL; ++k)
 #pragma unroll
@@ -1313,9 +1323,12 @@ __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, con
 // empty (FLT_MAX, MAX_INDEX) pair (merge_path's condition for its split
 // search).
 // BIG: pbeam > 256 (the merge-path with two or more segments per lane).
-template <bool BIG, int NW = 1>
+// SPLIT (BIG only): run by both waves of a team (wave wv), which sort alike and
+// share the segments; the last of three meetings ends it.
+template <bool BIG, int NW = 1, bool SPLIT = false>
 __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uint2 *ms, const float *cd,
-                                           const uint32_t *ci, int span, bool &fast_ok, int &lb_out) {
+                                           const uint32_t *ci, int span, bool &fast_ok, int &lb_out, int wv = 0) {
+    static_assert(!SPLIT || BIG, "split merge");
     const int lane = lane_id_opaque();
     lb_out = 0;
     const int nl = lane & 31;
@@ -1325,6 +1338,9 @@ __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uin
     const bool clean =
         !any_lane(!(((ck > -FLT_MAX) & (ck < FLT_MAX) & (cv != kMaxIndex)) | ((ck == FLT_MAX) & (cv == kMaxIndex))));
     fast_ok = fast_ok && clean;
+    // (both waves have read the candidates before either writes them sorted;
+    // they write the same pairs)
+    if constexpr (SPLIT) __syncthreads();
     sort_to(ms, ck, cv, span, clean);
     lead_sync<NW>();
     if constexpr (!BIG) {
@@ -1335,7 +1351,7 @@ __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uin
         } else if (pbeam == 32) {
             small_merge<1, true>(pbeam, bp, ms, nl, lane < 32);
         } else {
-            merge_path<1, NW>(P, bp, ms, fast_ok, 0);  // one segment per lane: nothing to save
+            merge_path<1, NW>(P, bp, ms, fast_ok, 0, P.seg_active);  // one segment per lane: nothing to save
         }
     } else {
         // Segments whose outputs lie wholly at or before position lb, the
@@ -1360,12 +1376,17 @@ __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uin
             return static_cast<int>(__umulhi(static_cast<uint32_t>(t * pbeam), P.seg_magic));
         };
         if (tf < active && seg_end(tf + 1) <= lb) ++tf;
-        const int spl = (active - tf + 63) / 64;
-        if (spl == 1) merge_path<1, NW>(P, bp, ms, fast_ok, tf);
-        else if (spl == 2) merge_path<2, NW>(P, bp, ms, fast_ok, tf);
-        else if (spl > 2) merge_path<4, NW>(P, bp, ms, fast_ok, tf);
+        // the team form's halves: [tf, mid) and [mid, active), the second
+        // from mid - 1 on for its first left boundary
+        const int mid = tf + (active - tf + 1) / 2;
+        const int t0 = SPLIT && wv ? mid - 1 : tf, t1 = SPLIT && !wv ? mid : active;
+        const int spl = tf < active ? (t1 - t0 + 63) / 64 : 0;
+        if (spl == 1) merge_path<1, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, SPLIT && wv);
+        else if (spl == 2) merge_path<2, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, SPLIT && wv);
+        else if (spl > 2) merge_path<4, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, SPLIT && wv);
     }
-    lead_sync<NW>();
+    if constexpr (SPLIT) __syncthreads();
+    else lead_sync<NW>();
 }
 
 // ------------------------------------------------------------ visited table
@@ -1445,10 +1466,10 @@ __device__ __forceinline__ uint32_t hash_insert(uint32_t *t, uint32_t nb, uint32
     return 0;
 }
 
-__device__ __forceinline__ void hash_reset(uint32_t *t, uint32_t nb) {
+__device__ __forceinline__ void hash_reset(uint32_t *t, uint32_t nb, int first, int step) {
     uint4 *t4 = reinterpret_cast<uint4 *>(t);
     const uint4 e = make_uint4(kMaxIndex, kMaxIndex, kMaxIndex, kMaxIndex);
-    for (uint32_t i = static_cast<uint32_t>(lane_id()); i < nb; i += 64) t4[i] = e;
+    for (uint32_t i = static_cast<uint32_t>(first); i < nb; i += static_cast<uint32_t>(step)) t4[i] = e;
 }
 
 // true iff an earlier (lower-lane) member of `members` in this half carries
@@ -1870,7 +1891,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
     // wave index within the team (0 for the one-wave form)
     const int wv = NW > 1 ? (__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x)) >> 6) : 0;
     const bool lead = NW == 1 || wv == 0;
-    TeamBlock *tb = reinterpret_cast<TeamBlock *>(smem + P.lds.team_off);
+    TeamBlock *tb = reinterpret_cast<TeamBlock *>(smem + P.lds.total);
     (void)tb;
     const int h = lane >> 5, nl = lane & 31;
     const Geo<DIM_T, DEG_T> g(P);
@@ -1885,7 +1906,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
     constexpr LdsLayout kL = lds_layout(DIM_T, Geo<DIM_T, DEG_T>::kB, 0, 0);
     const uint32_t msort_off = kFixedGeo ? kL.msort_off : P.lds.msort_off;
     const uint32_t scratch_off = kFixedGeo ? kL.scratch_off : P.lds.scratch_off;
-    const uint32_t prof_off = P.lds.prof_off;
+    const uint32_t prof_off = NW > 1 ? P.lds.total_team : P.lds.total;
     static_assert(kL.prep_off == 0u, "fixed LDS regions");
     uint32_t *H = reinterpret_cast<uint32_t *>(smem + P.lds.hash_off);
     // beam pairs: bp[-1] and bp[pbeam] are sentinels
@@ -1955,7 +1976,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                                                  P.use_ip != 0, true)));
 
         // ---- state (adaptive_search.cuh:67-107)
-        hash_reset(H, nbk);
+        hash_reset(H, nbk, lane, 64);
         for (int i = lane - 1; i < P.pbeam + static_cast<int>(kBeamPad); i += 64) bp[i] = i < 0 ? kLowSentinel : kEmpty;
         if (lane <= kMsortHi + 1) ms[lane - 1] = lane == 0 ? kLowSentinel : kEmpty;  // candidates empty
         lead_sync<NW>();
@@ -2065,14 +2086,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
         float kth = FLT_MAX, rho = 0.0f;
         int theta = 1;
         uint32_t nexp = 0;
+        if (((iter + 1) % kHashReset) == 0) {  // adaptive_search.cuh:128-134
+            // (a team's waves take half each; the second meeting is before the
+            // merge, which rewrites the beam they read)
+            const int tid = NW > 1 ? lane + 64 * wv : lane;
+            hash_reset(H, nbk, tid, 64 * NW);
+            if constexpr (NW > 1) __syncthreads();
+            else lead_sync<NW>();
+            for (int i = tid; i < beam_sz; i += 64 * NW) hash_insert(H, nbk, bp[i].y & ~kMsb);
+            if constexpr (NW > 1) __syncthreads();
+            else lead_sync<NW>();
+        }
+        FG_PHASE(1);
+        constexpr bool kSplitMerge = BIG && NW > 1;
+        if constexpr (kSplitMerge)
+            merge_beam<BIG, NW, true>(P, bp, ms, cd, ci, cand_span, split_fast, lb_merge, wv);
         if (lead) {
-            if (((iter + 1) % kHashReset) == 0) {  // adaptive_search.cuh:128-134
-                hash_reset(H, nbk);
-                lead_sync<NW>();
-                for (int i = lane; i < beam_sz; i += 64) hash_insert(H, nbk, bp[i].y & ~kMsb);
-                lead_sync<NW>();
-            }
-            FG_PHASE(1);
             // The merge runs before the iteration-limit test, so a search stopped
             // by max_iter merges its last candidates here (the reference's final
             // merge, adaptive_search.cuh:447-451).  A search that stops because no
@@ -2081,7 +2110,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             // A search that runs all kMaxIterations iterations (max_iter > 1024,
             // i.e. beam >= 931) leaves the loop without passing here again and
             // merges after it.
-            merge_beam<BIG, NW>(P, bp, ms, cd, ci, cand_span, split_fast, lb_merge);
+            if constexpr (!kSplitMerge) merge_beam<BIG, NW>(P, bp, ms, cd, ci, cand_span, split_fast, lb_merge);
             if constexpr (BIG) scan_from = min(scan_from, lb_merge);
             FG_PHASE(2);
             if (iter >= P.max_iter) {
@@ -2499,57 +2528,40 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 select_smallest<G, SRN>(est, rest, rounds, maxk, kept);
 #pragma unroll
                 for (int sr = 0; sr < SRN; ++sr) klm[sr] = group_join<G>(kept[sr]);
-                // the kept lanes of all sub-rounds; in the team form the
-                // helper's half reaches the lead wave through LDS
-                uint64_t klmA[SR];
-                uint32_t cidA[SR];
+                // (e) kept children listed in (task, lane) order: a sub-round's
+                // TPW tasks sit in lane order and follow each other, so a kept
+                // lane's place is the running total plus its rank among the
+                // kept lanes of the wave.  A lane with nothing to list, and one
+                // past the 32nd place, writes the beam's pad entry that takes
+                // the merge's unused slots: no branch.  The helper's tasks
+                // follow the lead wave's: it lists its own, and the lead wave
+                // reads both lists.
+                uint32_t total = 0;
+                {
+                    uint32_t *list = lead ? alist : tb->list;
+                    const uint32_t spare =
+                        static_cast<uint32_t>(reinterpret_cast<uint32_t *>(bp + pbeam + 2) - list);
 #pragma unroll
-                for (int sr = 0; sr < SRN; ++sr) {
-                    klmA[sr] = klm[sr];
-                    cidA[sr] = cid[sr];
+                    for (int sr = 0; sr < SRN; ++sr) {
+                        const uint32_t e = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(klm[sr] >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(klm[sr]), total));
+                        list[(lane_in(klm[sr]) & (e < 32u)) ? e : spare] = cid[sr];
+                        total += static_cast<uint32_t>(__popcll(klm[sr]));
+                    }
                 }
+                uint32_t own = total;
                 if constexpr (NW > 1) {
-                    if (!lead) {
-#pragma unroll
-                        for (int sr = 0; sr < SRN; ++sr) {
-                            if (lane == 0) tb->klm[sr] = klm[sr];
-                            tb->cid[sr][lane] = cid[sr];
-                        }
-                    }
+                    if (!lead && lane == 0) tb->n_list = total;
                     __syncthreads();
-                    if (lead) {
-#pragma unroll
-                        for (int sr = 0; sr < SRN; ++sr) {
-                            const uint64_t m = tb->klm[sr];
-                            klmA[SRN + sr] = (static_cast<uint64_t>(uni(static_cast<uint32_t>(m >> 32))) << 32) |
-                                             uni(static_cast<uint32_t>(m));
-                            cidA[SRN + sr] = tb->cid[sr][lane];
-                        }
-                    }
+                    if (lead) total += uni(tb->n_list);
                 }
                 if (lead) {
-                    // (e) kept children listed in (task, lane) order
-                    uint32_t total = 0;
-                    const uint32_t list_spare =
-                        (P.lds.beam_off + 8u * static_cast<uint32_t>(pbeam + 3) - scratch_off) / 4u;
-#pragma unroll
-                    for (int sr = 0; sr < SR; ++sr) {
-                        // the sub-round's TPW tasks sit in lane order and follow
-                        // each other in the list: a kept lane's place is the running
-                        // total plus its rank among the kept lanes of the wave
-                        // (a lane with nothing to list, and one past the 32nd
-                        // place, writes the beam's pad entry that takes the
-                        // merge's unused slots: no branch)
-                        const uint32_t e = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(klmA[sr] >> 32),
-                                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(klmA[sr]), total));
-                        alist[(lane_in(klmA[sr]) & (e < 32u)) ? e : list_spare] = cidA[sr];
-                        total += static_cast<uint32_t>(__popcll(klmA[sr]));
-                    }
                     lead_sync<NW>();
                     if (total > 32) total = 32;  // <= 4 kept per task at theta = 8
                     // (f) insert in list order; a repeat of an earlier entry is dropped
                     const bool mine = lane < static_cast<int>(total);
-                    const uint32_t key = mine ? alist[lane] : kMaxIndex;
+                    const uint32_t *from = NW > 1 && lane >= static_cast<int>(own) ? tb->list + (lane - own) : alist + lane;
+                    const uint32_t key = mine ? *from : kMaxIndex;
                     const uint32_t got = mine ? hash_insert(H, nbk, key) : 0u;
                     // Every listed child was absent from the table when this
                     // round's visited tests ran, so an insert that finds its key
@@ -2596,6 +2608,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             }
             __syncthreads();
             const int n_all = static_cast<int>(uni(tb->ex_n));
+            if (!lead) cand_span = theta <= 1 ? 32 : n_all;  // (the lead wave's, for the split merge)
             const uint32_t *lst = uni(tb->ex_alist) != 0u ? alist : nullptr;
             const int mid = (n_all + 1) >> 1;
             exact_batch_range<DPL>(P, g, lead ? 0 : mid, lead ? mid : n_all, lst, cd, ci, qr, qsrc);
@@ -2692,32 +2705,35 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
     }
 }
 
-// Whether a launch runs the team form: when the batch is too small to fill
-// the device with one wave per query (twice the queries fit in the
-// one-wave form's resident workgroups), a second wave per query costs no
-// query a slot and shortens every search.  FLASHGANN_TEAM=0 / 1 forces the
-// one-wave / team form (tests run both).
-// Workgroups of the one-wave kernel the device holds at once (0 if unknown).
-inline long long resident_one_wave(const SearchParams &P, const void *one_wave_kernel) {
+// Workgroups of a kernel the device holds at once (0 if unknown).
+inline long long resident_groups(const void *kernel, int threads, uint32_t lds) {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, one_wave_kernel, 64, P.lds.total) != hipSuccess) return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, lds) != hipSuccess) return 0;
     return static_cast<long long>(per_cu) * cus;
 }
 
-inline bool use_team(const SearchParams &P, const void *one_wave_kernel) {
+// Whether a launch runs the team form: when a second wave per query costs no
+// query a slot.  That is when the device holds the whole batch in the team
+// form, and when it holds (nearly) as many queries in either form, which is
+// where LDS, not registers, bounds them: at beam 1024 ten queries a CU, two
+// and a half waves a SIMD in the one-wave form, its vector units idle for 60%
+// of the time (d 128, 10,000 queries at beam 1024 in the one-wave form's two
+// launches 6.7 ms, in the team form 5.94; 2,000 queries 1.75 and 1.61; 3,000
+// queries at beam 256 0.66 and 0.635).  Where the second wave does cost
+// slots the one-wave form is faster (10,000 queries at beam 256: +19% in the
+// team form).
+// FLASHGANN_TEAM=0 / 1 forces the one-wave / team form (tests run both).
+inline bool use_team(const SearchParams &P, const void *one_wave_kernel, const void *team_kernel) {
     if (!P.team) return false;
     if (const char *e = std::getenv("FLASHGANN_TEAM")) {
         if (e[0] == '0') return false;
         if (e[0] == '1') return true;
     }
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return false;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, one_wave_kernel, 64, P.lds.total) != hipSuccess)
-        return false;
-    return 2ll * P.nq <= static_cast<long long>(per_cu) * cus;
+    const long long team = resident_groups(team_kernel, 128, P.lds.total_team);
+    if (P.nq <= team) return true;
+    return 10 * team >= 9 * resident_groups(one_wave_kernel, 64, P.lds.total);
 }
 
 template <int WT, int DPL, int DIM_T, int DEG_T, bool BIG>
@@ -2725,17 +2741,18 @@ void launch_geo_b(const SearchParams &P, hipStream_t stream, bool count, bool pr
                   long long *resident) {
     const dim3 grid(P.nq), block(64);
     const void *one = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 1>);
-    const bool team = !one_wave && use_team(P, one);
+    const void *two = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 2>);
+    const bool team = !one_wave && use_team(P, one, two);
     if (waves_only) {  // the form only, no launch
         *waves_only = team ? 2 : 1;
-        if (resident) *resident = resident_one_wave(P, one);
+        if (resident) *resident = resident_groups(one, 64, P.lds.total);
         return;
     }
     if (team) {
         const dim3 team_block(128);
         if (prof)
             hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, true, BIG, 2>), grid, team_block,
-                               P.lds.total_team, stream, P);
+                               P.lds.total_team + kProfBytes, stream, P);
         else if (count)
             hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, true, false, BIG, 2>), grid, team_block,
                                P.lds.total_team, stream, P);
@@ -2746,7 +2763,7 @@ void launch_geo_b(const SearchParams &P, hipStream_t stream, bool count, bool pr
     }
     if (prof)
         hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, true, BIG, 1>), grid, block,
-                           P.lds.total_prof, stream, P);
+                           P.lds.total + kProfBytes, stream, P);
     else if (count)
         hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, true, false, BIG, 1>), grid, block, P.lds.total,
                            stream, P);

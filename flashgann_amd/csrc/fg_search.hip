@@ -6,7 +6,7 @@
 //   * one workgroup = one wave = one query; the reference's 256-thread block
 //     barriers become wave-ordered LDS traffic, so the beam, candidate buffer,
 //     visited table and controller state never leave the CU's LDS/registers
-//     (a launch too small to fill the device runs the team form instead: a
+//     (where a second wave costs no query a slot the team form runs instead: a
 //     second wave per query takes half of the expansion rounds and of the
 //     exact distances);
 //   * the reference's 32-lane sorting networks are data-oblivious, so the

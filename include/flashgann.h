@@ -166,9 +166,11 @@ int fg_search_profile(fg_index *index, const float *d_queries, uint32_t nq, uint
 uint32_t fg_lds_bytes(uint32_t dim, uint32_t beam, uint32_t degree);
 
 /* Waves per query (1 or 2) that a search of nq queries at this K and beam
- * launches on the current device: two, the kernel's team form, when the batch
- * is too small to fill the device with one wave per query; FLASHGANN_TEAM=0/1
- * in the environment forces one form.  Results are identical either way.
+ * launches on the current device: two, the kernel's team form, when a second
+ * wave per query costs no query a slot (the device holds the whole batch in
+ * the team form, or, at wide beams, as many queries in either form);
+ * FLASHGANN_TEAM=0/1 in the environment forces one form.  Results are
+ * identical either way.
  * Negative FG_E* on invalid arguments.  No counterpart in the reference (one
  * warp-per-parent block shape). */
 int fg_search_waves(fg_index *index, uint32_t nq, uint32_t K, uint32_t beam);
