@@ -581,6 +581,10 @@ struct fg_index {
     size_t res_cap = 0;
     uint32_t *d_cnt = nullptr;
     size_t cnt_cap = 0;
+    // small host searches: a page-locked block that the kernel reads queries
+    // from and writes ids to (kHostStage bytes, allocated on first use), and
+    // its device address
+    unsigned char *h_stage = nullptr, *h_stage_dev = nullptr;
     // two-launch search: suspended queries' state, keys and order; the event
     // after the last sliced search, which the next one waits for
     uint32_t *d_slice = nullptr;
@@ -1093,6 +1097,7 @@ void fg_index_destroy(fg_index *ix) {
     if (ix->d_q) (void)hipFree(ix->d_q);
     if (ix->d_res) (void)hipFree(ix->d_res);
     if (ix->d_cnt) (void)hipFree(ix->d_cnt);
+    if (ix->h_stage) (void)hipHostFree(ix->h_stage);
     if (ix->slice_done) (void)hipEventDestroy(ix->slice_done);
     if (ix->d_slice) (void)hipFree(ix->d_slice);
     if (ix->ev0) (void)hipEventDestroy(ix->ev0);
@@ -1210,20 +1215,10 @@ int fg_search_profile(fg_index *ix, const float *d_queries, uint32_t nq, uint32_
 
 namespace {
 
-// Host-buffer search of fg_search / fg_search_noalloc: the queries are copied
-// into `dq`, the kernel runs on the null stream, and the ids (and counters)
-// are copied back from `dres` (`dcnt`).
-int search_host(fg_index *ix, SearchParams &P, const float *queries, uint32_t nq, uint32_t K, uint32_t *result_ids,
-                uint32_t *counters, fg_stats *stats, float *dq, uint32_t *dres, uint32_t *dcnt, bool may_slice) {
-    const size_t qb = static_cast<size_t>(nq) * ix->dim * sizeof(float);
-    const size_t rb = static_cast<size_t>(nq) * K * sizeof(uint32_t);
-    const size_t cb = static_cast<size_t>(nq) * FG_COUNTERS_PER_QUERY * sizeof(uint32_t);
-    FG_HIP(hipMemcpy(dq, queries, qb, hipMemcpyHostToDevice), "query upload");
+// The timed part of a host-buffer search (the reference's `elapsed`,
+// gpu_search_adaptive.cu:98-107): launch and synchronise.
+int search_timed(fg_index *ix, SearchParams &P, fg_stats *stats, bool may_slice) {
     FG_HIP(hipDeviceSynchronize(), "sync before search");
-    P.queries = dq;
-    P.results = dres;
-    P.counters = counters ? dcnt : nullptr;
-    P.phase = nullptr;
     const auto t0 = std::chrono::high_resolution_clock::now();
     FG_HIP(hipEventRecord(ix->ev0, nullptr), "event record");
     if (int rc = launch(ix, P, nullptr, may_slice)) return rc;
@@ -1235,9 +1230,70 @@ int search_host(fg_index *ix, SearchParams &P, const float *queries, uint32_t nq
         float ms = 0.0f;
         if (hipEventElapsedTime(&ms, ix->ev0, ix->ev1) == hipSuccess) stats->kernel_ms = ms;
     }
+    return FG_OK;
+}
+
+// Host-buffer search of fg_search / fg_search_noalloc: the queries are copied
+// into `dq`, the kernel runs on the null stream, and the ids (and counters)
+// are copied back from `dres` (`dcnt`).
+int search_host(fg_index *ix, SearchParams &P, const float *queries, uint32_t nq, uint32_t K, uint32_t *result_ids,
+                uint32_t *counters, fg_stats *stats, float *dq, uint32_t *dres, uint32_t *dcnt, bool may_slice) {
+    const size_t qb = static_cast<size_t>(nq) * ix->dim * sizeof(float);
+    const size_t rb = static_cast<size_t>(nq) * K * sizeof(uint32_t);
+    const size_t cb = static_cast<size_t>(nq) * FG_COUNTERS_PER_QUERY * sizeof(uint32_t);
+    FG_HIP(hipMemcpy(dq, queries, qb, hipMemcpyHostToDevice), "query upload");
+    P.queries = dq;
+    P.results = dres;
+    P.counters = counters ? dcnt : nullptr;
+    P.phase = nullptr;
+    if (int rc = search_timed(ix, P, stats, may_slice)) return rc;
     FG_HIP(hipMemcpy(result_ids, dres, rb, hipMemcpyDeviceToHost), "result download");
     if (counters) FG_HIP(hipMemcpy(counters, dcnt, cb, hipMemcpyDeviceToHost), "counter download");
     return FG_OK;
+}
+
+// A small host-buffer search: the kernel reads the queries from page-locked
+// host memory (once per query: padded dimensions up to 256 keep a query in
+// registers) and writes the ids there, so the call makes no copy of its own.
+// Each copy is a blocking call of some 15 us for any size: one query at d 128,
+// beam 64 took 156 us with them and takes 122, 256 queries at K 100 403 and 352.
+// The line at kHostStage is where copying through the
+// block on the host costs about what the device's copies do.
+constexpr size_t kHostStage = 256u << 10;
+
+int search_host_small(fg_index *ix, SearchParams &P, const float *queries, size_t qb, size_t rb, size_t cb,
+                      uint32_t *result_ids, uint32_t *counters, fg_stats *stats) {
+    std::memcpy(ix->h_stage, queries, qb);
+    const size_t ro = align256(qb), co = ro + align256(rb);
+    P.queries = reinterpret_cast<const float *>(ix->h_stage_dev);
+    P.results = reinterpret_cast<uint32_t *>(ix->h_stage_dev + ro);
+    P.counters = counters ? reinterpret_cast<uint32_t *>(ix->h_stage_dev + co) : nullptr;
+    P.phase = nullptr;
+    if (int rc = search_timed(ix, P, stats, true)) return rc;
+    std::memcpy(result_ids, ix->h_stage + ro, rb);
+    if (counters) std::memcpy(counters, ix->h_stage + co, cb);
+    return FG_OK;
+}
+
+// Whether a search of these sizes takes that way, with its block in place (a
+// block that cannot be had leaves the search to the copying way).
+bool host_stage_fits(fg_index *ix, size_t qb, size_t rb, size_t cb) {
+    if (ix->padded_dim > 256u || align256(qb) + align256(rb) + cb > kHostStage) return false;
+    if (!ix->h_stage) {
+        void *h = nullptr, *d = nullptr;
+        if (hipHostMalloc(&h, kHostStage, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipHostFree(h);
+            return false;
+        }
+        ix->h_stage = static_cast<unsigned char *>(h);
+        ix->h_stage_dev = static_cast<unsigned char *>(d);
+    }
+    return true;
 }
 
 int search_prologue(fg_index *ix, const float *queries, uint32_t nq, uint32_t K, uint32_t beam, uint32_t *result_ids,
@@ -1266,6 +1322,8 @@ int fg_search(fg_index *ix, const float *queries, uint32_t nq, uint32_t K, uint3
     const size_t qb = static_cast<size_t>(nq) * ix->dim * sizeof(float);
     const size_t rb = static_cast<size_t>(nq) * K * sizeof(uint32_t);
     const size_t cb = static_cast<size_t>(nq) * FG_COUNTERS_PER_QUERY * sizeof(uint32_t);
+    if (host_stage_fits(ix, qb, rb, counters ? cb : 0))
+        return search_host_small(ix, P, queries, qb, rb, cb, result_ids, counters, stats);
     if (int rc = ensure(reinterpret_cast<void **>(&ix->d_q), &ix->q_cap, qb)) return rc;
     if (int rc = ensure(reinterpret_cast<void **>(&ix->d_res), &ix->res_cap, rb)) return rc;
     if (counters)
