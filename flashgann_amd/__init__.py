@@ -129,7 +129,7 @@ class Index:
                                      C.c_void_p(stream or None)))
 
     def search_waves(self, nq: int, K: int, beam: int) -> int:
-        """Waves per query (1, or 2 for the kernel's team form) that a search
+        """Waves per query (1, or 2 or 4 for the kernel's team form) that a search
         of nq queries at this K and beam launches (fg_search_waves)."""
         w = lib().fg_search_waves(self._h, nq, K, beam)
         check(w if w < 0 else 0)

@@ -143,23 +143,23 @@ constexpr uint32_t kMsortPairs = 37;
 // slots are written to pbeam + 2).
 constexpr uint32_t kBeamPad = 4;
 
-// A team launch runs each query on two waves: the lead wave runs the search;
-// the helper takes half of every stage-II round (visited tests, estimates
-// and keep decisions of its tasks), half of every exact-distance batch, half
-// of every visited-table rebuild and, at beams over 256, half of the merge's
-// segments.  They meet at workgroup barriers and exchange through this LDS
-// block.
+// A team launch runs each query on two waves, or on four for wide vectors: the
+// lead wave runs the search; the helpers take their share of every stage-II
+// round (visited tests, estimates and keep decisions of their tasks), of every
+// exact-distance batch, of every visited-table rebuild and, at beams over 256,
+// of the merge's segments.  They meet at workgroup barriers and exchange
+// through this LDS block.
 struct TeamBlock {
     // per iteration, from the lead wave: stop flag, theta, rho, K-th cutoff,
     // number of expanders; then the exact batch's size and list kind
     uint32_t stop, theta, nexp, kth_bits, rho_bits, ex_n, ex_alist;
     // per query (written once): the quantised query's constants
     uint32_t sum_q, qwidth_bits, qlow_bits, any_wrap;
-    // the helper's work counters (counting build)
-    uint32_t c_ids, c_est;
-    // the helper's stage-II results: the kept children of its sub-rounds, in
-    // (task, lane) order (at most 4 per task at theta = 8)
-    uint32_t n_list;
+    // the helpers' stage-II results: the kept children of their sub-rounds, in
+    // (task, lane) order: at most 4 per task at theta = 8, so 16 from the
+    // one helper of two waves, 8 from each of the three of four; and, at the
+    // end, their work counters (counting build)
+    uint32_t n_list[3];
     uint32_t list[32];
 };
 constexpr uint32_t kTeamBytes = 192;
@@ -1166,10 +1166,10 @@ __device__ __forceinline__ void small_merge(int pbeam, uint2 *bp, const uint2 *m
 // split of such a tie gives the same output.  Any other equal pair sends the
 // whole wave through the reference's bisection, replayed step by step.
 //
-// SPLIT: both waves of a team take part, each with its own range of segments
-// (tbase, active); the waves meet between the reads and the writes.  The
-// second wave's range starts one segment early, for that segment's right
-// boundary alone (`shadow`: it is not written).
+// SPLIT: every wave of a team takes part, each with its own range of segments
+// (tbase, active); the waves meet between the reads and the writes.  A range
+// after the first starts one segment early, for that segment's right boundary
+// alone (`shadow`: it is not written).
 template <int SPL, int NW = 1, bool SPLIT = false>
 __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, const uint2 *ms, bool fast_ok, int tbase,
                                            int active, bool shadow = false) {
@@ -1323,7 +1323,7 @@ __device__ __forceinline__ void merge_path(const SearchParams &P, uint2 *bp, con
 // empty (FLT_MAX, MAX_INDEX) pair (merge_path's condition for its split
 // search).
 // BIG: pbeam > 256 (the merge-path with two or more segments per lane).
-// SPLIT (BIG only): run by both waves of a team (wave wv), which sort alike and
+// SPLIT (BIG only): run by every wave of a team (wave wv), which sort alike and
 // share the segments; the last of three meetings ends it.
 template <bool BIG, int NW = 1, bool SPLIT = false>
 __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uint2 *ms, const float *cd,
@@ -1338,8 +1338,8 @@ __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uin
     const bool clean =
         !any_lane(!(((ck > -FLT_MAX) & (ck < FLT_MAX) & (cv != kMaxIndex)) | ((ck == FLT_MAX) & (cv == kMaxIndex))));
     fast_ok = fast_ok && clean;
-    // (both waves have read the candidates before either writes them sorted;
-    // they write the same pairs)
+    // (every wave has read the candidates before any writes them sorted; they
+    // write the same pairs)
     if constexpr (SPLIT) __syncthreads();
     sort_to(ms, ck, cv, span, clean);
     lead_sync<NW>();
@@ -1376,14 +1376,16 @@ __device__ __forceinline__ void merge_beam(const SearchParams &P, uint2 *bp, uin
             return static_cast<int>(__umulhi(static_cast<uint32_t>(t * pbeam), P.seg_magic));
         };
         if (tf < active && seg_end(tf + 1) <= lb) ++tf;
-        // the team form's halves: [tf, mid) and [mid, active), the second
-        // from mid - 1 on for its first left boundary
-        const int mid = tf + (active - tf + 1) / 2;
-        const int t0 = SPLIT && wv ? mid - 1 : tf, t1 = SPLIT && !wv ? mid : active;
-        const int spl = tf < active ? (t1 - t0 + 63) / 64 : 0;
-        if (spl == 1) merge_path<1, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, SPLIT && wv);
-        else if (spl == 2) merge_path<2, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, SPLIT && wv);
-        else if (spl > 2) merge_path<4, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, SPLIT && wv);
+        // a team's waves take equal ranges; each after the first starts one
+        // segment early, for its first left boundary
+        const int per = SPLIT ? (active - tf + NW - 1) / NW : active - tf;
+        const int t0 = SPLIT && wv ? tf + wv * per - 1 : tf, t1 = SPLIT ? min(tf + (wv + 1) * per, active) : active;
+        const bool shadow = SPLIT && wv;
+        const int spl = t0 + (shadow ? 1 : 0) < t1 ? (t1 - t0 + 63) / 64 : 0;
+        if (spl == 1) merge_path<1, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, shadow);
+        else if (spl == 2) merge_path<2, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, shadow);
+        else if (spl > 2) merge_path<4, NW, SPLIT>(P, bp, ms, fast_ok, t0, t1, shadow);
+        else if (SPLIT && tf < active) __syncthreads();  // a wave without segments joins the others' meeting
     }
     if constexpr (SPLIT) __syncthreads();
     else lead_sync<NW>();
@@ -1865,13 +1867,13 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
 // it keeps in flight: at padded dimension 2048 its LDS (digit rows, rotation
 // scratch) holds it to 3 waves per SIMD anyway, and at 1024 a
 // 1,000-query launch fills one wave per SIMD.
-// NW = 2: the team form (two waves per query; see TeamBlock).  Wave 0 leads:
+// NW = 2 or 4: the team form (two or four waves per query; see TeamBlock).  Wave 0 leads:
 // it runs every phase, the helper wave joins it in stage II's rounds and the
 // exact distances; `lead_sync` orders the lead wave's own LDS accesses and
 // the workgroup barriers mark the meeting points.
 template <int WT, int DPL, int DIM_T, int DEG_T, bool COUNT, bool PROF, bool BIG, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? 3 : WT > 4 ? 4 : 5))) void fg_search_kernel(SearchParams P) {
-    static_assert(NW == 1 || NW == 2, "team form: two waves");
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : 5))) void fg_search_kernel(SearchParams P) {
+    static_assert(NW == 1 || NW == 2 || (NW == 4 && WT == 0), "team form: two waves, four for wide vectors");
     extern __shared__ __align__(16) unsigned char smem[];
     int qid = blockIdx.x;
     if (qid >= P.nq) return;
@@ -2538,29 +2540,45 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 // reads both lists.
                 uint32_t total = 0;
                 {
-                    uint32_t *list = lead ? alist : tb->list;
+                    constexpr int kHelpers = NW > 1 ? NW - 1 : 1;
+                    constexpr uint32_t kRoom = NW > 2 ? 8u : 32u;  // of a helper's list
+                    static_assert(kHelpers * kRoom <= 32u, "team lists");
+                    uint32_t *list = lead ? alist : tb->list + kRoom * static_cast<uint32_t>(wv - 1);
+                    const uint32_t room = lead ? 32u : kRoom;
                     const uint32_t spare =
                         static_cast<uint32_t>(reinterpret_cast<uint32_t *>(bp + pbeam + 2) - list);
 #pragma unroll
                     for (int sr = 0; sr < SRN; ++sr) {
                         const uint32_t e = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(klm[sr] >> 32),
                                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(klm[sr]), total));
-                        list[(lane_in(klm[sr]) & (e < 32u)) ? e : spare] = cid[sr];
+                        list[(lane_in(klm[sr]) & (e < room)) ? e : spare] = cid[sr];
                         total += static_cast<uint32_t>(__popcll(klm[sr]));
                     }
                 }
-                uint32_t own = total;
+                // ends of the lead wave's list and the helpers'
+                uint32_t ends[NW];
+                ends[0] = total;
                 if constexpr (NW > 1) {
-                    if (!lead && lane == 0) tb->n_list = total;
+                    if (!lead && lane == 0) tb->n_list[wv - 1] = total;
                     __syncthreads();
-                    if (lead) total += uni(tb->n_list);
+                    if (lead) {
+#pragma unroll
+                        for (int i = 1; i < NW; ++i) ends[i] = ends[i - 1] + uni(tb->n_list[i - 1]);
+                        total = ends[NW - 1];
+                    }
                 }
                 if (lead) {
                     lead_sync<NW>();
                     if (total > 32) total = 32;  // <= 4 kept per task at theta = 8
                     // (f) insert in list order; a repeat of an earlier entry is dropped
                     const bool mine = lane < static_cast<int>(total);
-                    const uint32_t *from = NW > 1 && lane >= static_cast<int>(own) ? tb->list + (lane - own) : alist + lane;
+                    const uint32_t *from = alist + lane;
+                    if constexpr (NW > 1) {
+#pragma unroll
+                        for (int i = 1; i < NW; ++i)
+                            if (lane >= static_cast<int>(ends[i - 1]))
+                                from = tb->list + (NW > 2 ? 8 : 32) * (i - 1) + (lane - static_cast<int>(ends[i - 1]));
+                    }
                     const uint32_t key = mine ? *from : kMaxIndex;
                     const uint32_t got = mine ? hash_insert(H, nbk, key) : 0u;
                     // Every listed child was absent from the table when this
@@ -2601,7 +2619,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
         if constexpr (NW == 1) {
             exact_batch<DPL>(P, g, ex_n, ex_list, cd, ci, qr, qsrc);
         } else {
-            // the exact batch in two halves, one per wave
+            // the exact batch in equal shares, one per wave
             if (lead && lane == 0) {
                 tb->ex_n = static_cast<uint32_t>(ex_n);
                 tb->ex_alist = ex_list != nullptr ? 1u : 0u;
@@ -2610,8 +2628,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             const int n_all = static_cast<int>(uni(tb->ex_n));
             if (!lead) cand_span = theta <= 1 ? 32 : n_all;  // (the lead wave's, for the split merge)
             const uint32_t *lst = uni(tb->ex_alist) != 0u ? alist : nullptr;
-            const int mid = (n_all + 1) >> 1;
-            exact_batch_range<DPL>(P, g, lead ? 0 : mid, lead ? mid : n_all, lst, cd, ci, qr, qsrc);
+            exact_batch_range<DPL>(P, g, n_all * wv / NW, n_all * (wv + 1) / NW, lst, cd, ci, qr, qsrc);
             __syncthreads();
         }
         if (theta <= 1) FG_PHASE(5);
@@ -2619,16 +2636,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
         lead_sync<NW>();
     }
     if constexpr (NW > 1) {
-        // the helper's work counters; from here on the lead wave is alone
+        // the helpers' work counters; from here on the lead wave is alone
         if (!lead && lane == 0) {
-            tb->c_ids = c_ids;
-            tb->c_est = c_est;
+            tb->list[2 * wv] = c_ids;
+            tb->list[2 * wv + 1] = c_est;
         }
         __syncthreads();
         if (!lead) return;
         if constexpr (COUNT) {
-            c_ids += uni(tb->c_ids);
-            c_est += uni(tb->c_est);
+#pragma unroll
+            for (int i = 1; i < NW; ++i) {
+                c_ids += uni(tb->list[2 * i]);
+                c_est += uni(tb->list[2 * i + 1]);
+            }
         }
     }
     if constexpr (kSliceable) {
@@ -2714,62 +2734,70 @@ inline long long resident_groups(const void *kernel, int threads, uint32_t lds) 
     return static_cast<long long>(per_cu) * cus;
 }
 
-// Whether a launch runs the team form: when a second wave per query costs no
-// query a slot.  That is when the device holds the whole batch in the team
-// form, and when it holds (nearly) as many queries in either form, which is
-// where LDS, not registers, bounds them: at beam 1024 ten queries a CU, two
-// and a half waves a SIMD in the one-wave form, its vector units idle for 60%
-// of the time (d 128, 10,000 queries at beam 1024 in the one-wave form's two
-// launches 6.7 ms, in the team form 5.94; 2,000 queries 1.75 and 1.61; 3,000
-// queries at beam 256 0.66 and 0.635).  Where the second wave does cost
-// slots the one-wave form is faster (10,000 queries at beam 256: +19% in the
-// team form).
-// FLASHGANN_TEAM=0 / 1 forces the one-wave / team form (tests run both).
-inline bool use_team(const SearchParams &P, const void *one_wave_kernel, const void *team_kernel) {
-    if (!P.team) return false;
-    if (const char *e = std::getenv("FLASHGANN_TEAM")) {
-        if (e[0] == '0') return false;
-        if (e[0] == '1') return true;
-    }
-    const long long team = resident_groups(team_kernel, 128, P.lds.total_team);
-    if (P.nq <= team) return true;
-    return 10 * team >= 9 * resident_groups(one_wave_kernel, 64, P.lds.total);
+// Waves per query of a launch: two, the team form, when a second wave per
+// query costs no query a slot.  That is when the device holds the whole batch
+// in the team form, and when it holds (nearly) as many queries in either form,
+// which is where LDS, not registers, bounds them: at beam 1024 ten queries a
+// CU, two and a half waves a SIMD in the one-wave form, its vector units idle
+// for 60% of the time (d 128, 10,000 queries at beam 1024 in the one-wave
+// form's two launches 6.7 ms, in the team form 5.94; 2,000 queries 1.75 and
+// 1.61; 3,000 queries at beam 256 0.66 and 0.635).  Where the second wave does
+// cost slots the one-wave form is faster (10,000 queries at beam 256: +19% in
+// the team form).  Four waves, for wide vectors (four_wave_kernel), when the
+// device holds the batch in that form too: there the stages that share out,
+// the estimates and exact distances, are most of an iteration (d 960, beam 384:
+// 1,000 queries 0.970 ms in two waves, 0.929 in four, 100 queries 0.763 and
+// 0.652; d 1536, beam 640: 64 queries 1.78 ms before and 1.18).
+// FLASHGANN_TEAM=0 / 1 forces the one-wave / a team form (tests run both).
+inline int team_waves(const SearchParams &P, const void *one_wave_kernel, const void *two_wave_kernel,
+                      const void *four_wave_kernel) {
+    if (!P.team) return 1;
+    const char *e = std::getenv("FLASHGANN_TEAM");
+    if (e && e[0] == '0') return 1;
+    if (four_wave_kernel && P.nq <= resident_groups(four_wave_kernel, 256, P.lds.total_team)) return 4;
+    if (e && e[0] == '1') return 2;
+    const long long team = resident_groups(two_wave_kernel, 128, P.lds.total_team);
+    if (P.nq <= team) return 2;
+    return 10 * team >= 9 * resident_groups(one_wave_kernel, 64, P.lds.total) ? 2 : 1;
+}
+
+template <int WT, int DPL, int DIM_T, int DEG_T, bool BIG, int NW>
+void launch_form(const SearchParams &P, hipStream_t stream, bool count, bool prof) {
+    const dim3 grid(P.nq), block(64 * NW);
+    const uint32_t lds = NW > 1 ? P.lds.total_team : P.lds.total;
+    if (prof)
+        hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, true, BIG, NW>), grid, block,
+                           lds + kProfBytes, stream, P);
+    else if (count)
+        hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, true, false, BIG, NW>), grid, block, lds, stream,
+                           P);
+    else
+        hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, NW>), grid, block, lds, stream,
+                           P);
 }
 
 template <int WT, int DPL, int DIM_T, int DEG_T, bool BIG>
 void launch_geo_b(const SearchParams &P, hipStream_t stream, bool count, bool prof, int *waves_only, bool one_wave,
                   long long *resident) {
-    const dim3 grid(P.nq), block(64);
     const void *one = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 1>);
     const void *two = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 2>);
-    const bool team = !one_wave && use_team(P, one, two);
+    const void *four = nullptr;
+    if constexpr (WT == 0)
+        four = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 4>);
+    const int waves = one_wave ? 1 : team_waves(P, one, two, four);
     if (waves_only) {  // the form only, no launch
-        *waves_only = team ? 2 : 1;
+        *waves_only = waves;
         if (resident) *resident = resident_groups(one, 64, P.lds.total);
         return;
     }
-    if (team) {
-        const dim3 team_block(128);
-        if (prof)
-            hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, true, BIG, 2>), grid, team_block,
-                               P.lds.total_team + kProfBytes, stream, P);
-        else if (count)
-            hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, true, false, BIG, 2>), grid, team_block,
-                               P.lds.total_team, stream, P);
-        else
-            hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 2>), grid, team_block,
-                               P.lds.total_team, stream, P);
-        return;
+    if constexpr (WT == 0) {
+        if (waves == 4) {
+            launch_form<WT, DPL, DIM_T, DEG_T, BIG, 4>(P, stream, count, prof);
+            return;
+        }
     }
-    if (prof)
-        hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, true, BIG, 1>), grid, block,
-                           P.lds.total + kProfBytes, stream, P);
-    else if (count)
-        hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, true, false, BIG, 1>), grid, block, P.lds.total,
-                           stream, P);
-    else
-        hipLaunchKernelGGL((fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 1>), grid, block, P.lds.total,
-                           stream, P);
+    if (waves == 2) launch_form<WT, DPL, DIM_T, DEG_T, BIG, 2>(P, stream, count, prof);
+    else launch_form<WT, DPL, DIM_T, DEG_T, BIG, 1>(P, stream, count, prof);
 }
 
 // Beams over 256 (two or more merge-path segments per lane, the pick's wide

@@ -165,10 +165,12 @@ int fg_search_profile(fg_index *index, const float *d_queries, uint32_t nq, uint
  * calculate_shared_mem_size, src/adaptive_search_utils.cuh:152-176). */
 uint32_t fg_lds_bytes(uint32_t dim, uint32_t beam, uint32_t degree);
 
-/* Waves per query (1 or 2) that a search of nq queries at this K and beam
+/* Waves per query (1, 2 or 4) that a search of nq queries at this K and beam
  * launches on the current device: two, the kernel's team form, when a second
  * wave per query costs no query a slot (the device holds the whole batch in
- * the team form, or, at wide beams, as many queries in either form);
+ * the team form, or, at wide beams, as many queries in either form), four for
+ * vectors of more than 256 dimensions when the device holds the batch in that
+ * form;
  * FLASHGANN_TEAM=0/1 in the environment forces one form.  Results are
  * identical either way.
  * Negative FG_E* on invalid arguments.  No counterpart in the reference (one

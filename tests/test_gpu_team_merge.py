@@ -1,6 +1,6 @@
-"""The team form's beam merge above 256 entries, which its two waves share: ids
+"""The team form's beam merge above 256 entries, which its two or four waves share: ids
 and work counters against the oracle at beams around the segment counts where
-the halves change size (an odd number of segments, one per lane, more than
+the shares change size (an odd number of segments, one per lane, more than
 128, the full 256), on integer data, whose equal distances also take the
 merge through its tie replay."""
 from __future__ import annotations
@@ -21,7 +21,7 @@ def test_team_merge_matches_oracle(gpu_available, monkeypatch, beam, dim, kind):
     monkeypatch.setenv("FLASHGANN_TEAM", "1")
     cb, q, _ = small_index(n=2500, nq=16, dim=dim, comps=10, degree=32, kind=kind)
     ix = Index.from_codebook(cb)
-    assert ix.search_waves(q.shape[0], 20, beam) == 2
+    assert ix.search_waves(q.shape[0], 20, beam) == (4 if dim > 256 else 2)
     ids, _, cnt = ix.search(q, 20, beam, counters=True)
     ix.close()
     rids, rcnt = O.OracleIndex.from_codebook(cb).search(q, 20, beam)
