@@ -685,10 +685,11 @@ __device__ __forceinline__ LevelRows level_rows(uint32_t W) {
 template <int NB, int NWD>
 __device__ __forceinline__ void raw_mfma(const uint32_t (&c)[NB][NWD], const unsigned char *prep, LevelRows lr, int w0,
                                          v4f (&acc)[NB]) {
-    // The query's rows are read GA words ahead of the products that take them
-    // (the barriers keep the compiler from sinking a read to its product, an
-    // LDS round trip a word).
-    constexpr int GA = NWD <= 4 ? NWD : (NB == 1 ? 4 : 2);
+    // The query's rows of a wide code are read GA words ahead of the products
+    // that take them (the barriers keep the compiler from sinking a read to its
+    // product, an LDS round trip a word); of a narrow one the compiler places
+    // them, which holds fewer registers.
+    constexpr int GA = NWD <= 4 ? (NB == 1 ? NWD : 1) : (NB == 1 ? 4 : 2);
     const unsigned char *at = prep + lr.at + static_cast<uint32_t>(w0) * lr.step;
     int4 cur[GA], nxt[GA];
 #pragma unroll
@@ -704,7 +705,7 @@ __device__ __forceinline__ void raw_mfma(const uint32_t (&c)[NB][NWD], const uns
                 nxt[i] = *reinterpret_cast<const int4 *>(at);
                 at += lr.step;
             }
-            __builtin_amdgcn_sched_barrier(0);
+            if (NWD > 4) __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int i = 0; i < GA; ++i) {
@@ -1860,19 +1861,18 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
     } while (0)
 
 // One wave per workgroup; the register budget targets 5 waves per SIMD
-// (<= 96 VGPRs; the fixed-geometry kernels use 77-79, which leaves room for
-// a sixth), which LDS also allows for beams up to 256 (6,144 bytes a
-// workgroup at beam 256).  The generic-geometry instantiation (padded dimension
-// >= 256) gets 3 (<= 168 VGPRs) for its wide code batches and the plane reads
-// it keeps in flight: at padded dimension 2048 its LDS (digit rows, rotation
-// scratch) holds it to 3 waves per SIMD anyway, and at 1024 a
-// 1,000-query launch fills one wave per SIMD.
+// (<= 96 VGPRs), 6 (<= 80) for the fixed geometries at beams up to 256, where
+// LDS allows 25 workgroups a CU (against 5 waves: d 128, beam 256, 40,000
+// queries 4.61 -> 4.44 ms, 5,500 0.933 -> 0.886, 10,000, whose time is its
+// longest queries', the same; d 96, 10,000 queries 1.004 -> 0.977).  Padded
+// dimension 256 gets 4, and the wide runtime geometry 3 (<= 168 VGPRs) for its
+// code batches: at padded dimension 2048 its LDS holds it to about 3 anyway.
 // NW = 2 or 4: the team form (two or four waves per query; see TeamBlock).  Wave 0 leads:
 // it runs every phase, the helper wave joins it in stage II's rounds and the
 // exact distances; `lead_sync` orders the lead wave's own LDS accesses and
 // the workgroup barriers mark the meeting points.
 template <int WT, int DPL, int DIM_T, int DEG_T, bool COUNT, bool PROF, bool BIG, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : 5))) void fg_search_kernel(SearchParams P) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : (DIM_T > 0 && NW == 1 && !PROF && !BIG ? 6 : 5)))) void fg_search_kernel(SearchParams P) {
     static_assert(NW == 1 || NW == 2 || (NW == 4 && WT == 0), "team form: two waves, four for wide vectors");
     extern __shared__ __align__(16) unsigned char smem[];
     int qid = blockIdx.x;
@@ -2286,8 +2286,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                     const float sk = nl < cbs ? dist : FLT_MAX;
                     const uint32_t sv = nl < cbs ? child : kMaxIndex;
                     // (the runtime geometry of padded dimension 64 and 128 has no
-                    // registers left for the counted sort here as well)
-                    const bool clean = (kFixedGeo || WT == 0 || WT > 4) &&
+                    // registers left for the counted sort here as well, and in
+                    // the one-wave fixed-geometry kernel of beams up to 256 it
+                    // would cost the sixth wave per SIMD)
+                    const bool clean = ((kFixedGeo && (NW > 1 || BIG)) || WT == 0 || WT > 4) &&
                                        !any_lane(!(((sk > -FLT_MAX) & (sk < FLT_MAX) & (sv != kMaxIndex)) |
                                                    ((sk == FLT_MAX) & (sv == kMaxIndex))));
                     sort_to(ms, sk, sv, 32, clean);
