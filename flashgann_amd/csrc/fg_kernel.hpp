@@ -1872,7 +1872,7 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
 // exact distances; `lead_sync` orders the lead wave's own LDS accesses and
 // the workgroup barriers mark the meeting points.
 template <int WT, int DPL, int DIM_T, int DEG_T, bool COUNT, bool PROF, bool BIG, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : (DIM_T > 0 && NW == 1 && !PROF && !BIG ? 6 : 5)))) void fg_search_kernel(SearchParams P) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : (DIM_T > 0 && NW == 1 && !COUNT && !PROF && !BIG ? 6 : 5)))) void fg_search_kernel(SearchParams P) {
     static_assert(NW == 1 || NW == 2 || (NW == 4 && WT == 0), "team form: two waves, four for wide vectors");
     extern __shared__ __align__(16) unsigned char smem[];
     int qid = blockIdx.x;
@@ -2122,79 +2122,75 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             for (int i = beam_sz + lane; i < pbeam; i += 64) bp[i] = kEmpty;
             ms[nl] = kEmpty;  // both halves store the same pair: no branch
             lead_sync<NW>();
-            kth = FLT_MAX;  // adaptive_search_utils.cuh:25-30
-            if (bp[beam_sz - 1].y != kMaxIndex) kth = __uint_as_float(bp[(P.K < beam_sz ? P.K : beam_sz) - 1].x);
-            kth = uni(kth);
-            controller_step(ctl, uni(bp[0].y), P.phase2_rho);
+            // The cutoff's, the controller's and the pick's reads go out
+            // together: one LDS round trip.  pick_expanders (utils.cuh:752-787)
+            // takes the first theta unexpanded entries; entry base + 64 k + l
+            // is on lane l (each read covers 64 consecutive entries), so index
+            // order is k, then lane.  Beams up to 256 are read whole; larger
+            // ones, where the first unexpanded entry sits about halfway down,
+            // 256 entries per step, from the first that can be unexpanded.  (One
+            // round trip where there were up to seven: 777 queries at d 200
+            // 0.495 -> 0.478 ms, 1,000 at d 128, beam 256 0.538 -> 0.526; full
+            // launches, where other waves cover the trips, within 0.5% at beam
+            // 256, -1.5% at 512.)
+            constexpr int kPick = 4;
+            const int chunks = BIG ? kPick : (beam_sz + 63) / 64;
+            uint2 pe[kPick];
+            int pbase = BIG ? scan_from : 0;
+#pragma unroll
+            for (int k = 0; k < kPick; ++k) {
+                const int j = pbase + 64 * k + lane;
+                pe[k] = bp[j < pbeam ? j : pbeam];  // unconditional read; bp[pbeam] is a sentinel
+            }
+            const uint2 last_e = bp[beam_sz - 1], kth_e = bp[(P.K < beam_sz ? P.K : beam_sz) - 1];
+            const uint32_t top_id = bp[0].y;
+            kth = uni(last_e.y != kMaxIndex ? pair_key(kth_e) : FLT_MAX);  // adaptive_search_utils.cuh:25-30
+            controller_step(ctl, uni(top_id), P.phase2_rho);
             theta = ctl.spec;
             rho = ctl.rho;
-
-            // pick_expanders (utils.cuh:752-787): first theta unexpanded entries
-            // the picked entries' ids and distances go straight to the parent
-            // lists (an unexpanded entry's id has the top bit clear)
-            // Beams up to 256: lane l reads entry base + l (64 per step).  Larger
-            // beams, where the first unexpanded entry sits about halfway down: 256
-            // entries per step, from the first entry that can be unexpanded.
             nexp = 0;
-            if constexpr (!BIG) {
-                for (int base = 0; base < beam_sz; base += 64) {
-                    const int j = base + lane;
-                    const uint2 e = bp[j < pbeam ? j : pbeam];  // unconditional read; bp[pbeam] is a sentinel
-                    const bool fresh = j < beam_sz && (e.y & kMsb) == 0;
-                    const uint64_t m = ballot(fresh);
-                    if (fresh) {
-                        const uint32_t r = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull))) + nexp;
-                        if (r < static_cast<uint32_t>(theta)) {
-                            pnode[r] = e.y;
-                            pdist[r] = __uint_as_float(e.x);
-                            bp[j].y = e.y | kMsb;
-                        }
-                    }
-                    nexp += static_cast<uint32_t>(__popcll(m));
-                    if (nexp >= static_cast<uint32_t>(theta)) {
-                        nexp = static_cast<uint32_t>(theta);
-                        break;
-                    }
-                }
-            } else {
-              int lastj = -1;  // the entry that took rank theta - 1
-              for (int base = scan_from; base < beam_sz; base += 256) {
-                // entry base + 64 k + l on lane l (each read covers 64
-                // consecutive entries); index order is k, then lane
-                uint2 e[4];
-                uint64_t m[4];
+            float lastd = 0.0f;        // the distance of the last entry picked so far, on the lane that picked it
+            uint64_t lastm = 0ull;     // that lane
+            int lastj = -1;            // (beams over 256) the entry that took rank theta - 1
+            for (;;) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int j = base + 64 * k + lane;
-                    e[k] = bp[j < pbeam ? j : pbeam];  // unconditional read; bp[pbeam] is a sentinel
-                    m[k] = ballot(j < beam_sz && (e[k].y & kMsb) == 0);
-                }
-                const uint64_t lt = (1ull << lane) - 1ull;
-                uint32_t before = nexp;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (lane_in(m[k])) {
-                        const uint32_t r = before + static_cast<uint32_t>(__popcll(m[k] & lt));
-                        if (r < static_cast<uint32_t>(theta)) {
-                            const int j = base + 64 * k + lane;
-                            pnode[r] = e[k].y;
-                            pdist[r] = __uint_as_float(e[k].x);
-                            bp[j].y = e[k].y | kMsb;
-                            if (r + 1 == static_cast<uint32_t>(theta)) lastj = j;
+                for (int k = 0; k < kPick; ++k) {
+                    if (k < chunks && nexp < static_cast<uint32_t>(theta)) {
+                        const int j = pbase + 64 * k + lane;
+                        // the picked entries' ids and distances go straight to the
+                        // parent lists (an unexpanded entry's id has the top bit clear)
+                        const uint64_t m = ballot((j < beam_sz) & ((pe[k].y & kMsb) == 0u));
+                        const uint32_t r = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), nexp));
+                        if (lane_in(m) & (r < static_cast<uint32_t>(theta))) {
+                            pnode[r] = pe[k].y;
+                            pdist[r] = pair_key(pe[k]);
+                            bp[j].y = pe[k].y | kMsb;
                         }
+                        const uint32_t total = nexp + static_cast<uint32_t>(__popcll(m));
+                        const uint32_t now = min(total, static_cast<uint32_t>(theta));
+                        if (now > nexp) {
+                            lastm = ballot(r + 1u == now) & m;
+                            lastd = pair_key(pe[k]);
+                            if (BIG && now == static_cast<uint32_t>(theta)) lastj = j;
+                        }
+                        nexp = now;
                     }
-                    before += static_cast<uint32_t>(__popcll(m[k]));
                 }
-                nexp = before;
-                if (nexp >= static_cast<uint32_t>(theta)) {
-                    nexp = static_cast<uint32_t>(theta);
-                    break;
+                if (!BIG || nexp >= static_cast<uint32_t>(theta)) break;
+                pbase += 64 * kPick;
+                if (pbase >= beam_sz) break;
+#pragma unroll
+                for (int k = 0; k < kPick; ++k) {
+                    const int j = pbase + 64 * k + lane;
+                    pe[k] = bp[j < pbeam ? j : pbeam];
                 }
-              }
-              // entries up to the last one picked are now all expanded
-              const uint64_t bl = ballot(lastj >= 0);
-              scan_from = bl ? __builtin_amdgcn_readlane(lastj, __builtin_ctzll(bl)) + 1 : beam_sz;
             }
+            if constexpr (BIG)
+                // entries up to the last one picked are now all expanded
+                scan_from = nexp >= static_cast<uint32_t>(theta)
+                                ? __builtin_amdgcn_readlane(lastj, __builtin_ctzll(lastm)) + 1
+                                : beam_sz;
             lead_sync<NW>();
             if (nexp == 0) {
                 team_stop<NW>(tb, lane);
@@ -2204,7 +2200,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             FG_COUNT(c_exp += nexp);
             // adaptive_search_utils.cuh:41-49
             ctl.last_e = finite_below_max(ctl.cur_e) ? ctl.cur_e : ctl.entry_d;
-            ctl.cur_e = uni(pdist[nexp - 1]);
+            ctl.cur_e = __int_as_float(
+                __builtin_amdgcn_readlane(__float_as_int(lastd), __builtin_ctzll(lastm)));
         }
         if constexpr (NW > 1) {
             if (lead && lane == 0) {
@@ -2287,9 +2284,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                     const uint32_t sv = nl < cbs ? child : kMaxIndex;
                     // (the runtime geometry of padded dimension 64 and 128 has no
                     // registers left for the counted sort here as well, and in
-                    // the one-wave fixed-geometry kernel of beams up to 256 it
-                    // would cost the sixth wave per SIMD)
-                    const bool clean = ((kFixedGeo && (NW > 1 || BIG)) || WT == 0 || WT > 4) &&
+                    // the one-wave fixed-geometry kernels of degree 32 it would
+                    // cost a wave per SIMD)
+                    const bool clean = ((kFixedGeo && (NW > 1 || DEG_T == 16)) || WT == 0 || WT > 4) &&
                                        !any_lane(!(((sk > -FLT_MAX) & (sk < FLT_MAX) & (sv != kMaxIndex)) |
                                                    ((sk == FLT_MAX) & (sv == kMaxIndex))));
                     sort_to(ms, sk, sv, 32, clean);
