@@ -566,6 +566,15 @@ __device__ __forceinline__ void prepare_query(const float *__restrict__ query, c
                               int B, float *rot, float *qv, uint32_t *prep, float &low_out,
                               float &high_out, float &width_out, int &sumq_out, uint8_t *qdump) {
     const int lane = lane_id();
+    // Element i sits on lane i & 63: the butterflies of distance 1 .. 32 pair
+    // lanes (cross-lane moves, no LDS), those of 64 and up two elements of
+    // one lane (LDS words that no other lane touches: no meeting between
+    // steps).  As seven LDS steps with a meeting and an index division each,
+    // preparation was 8,000 cycles at d 128 and 70,000 at d 960: @MEAS5@.
+    const auto pair = [lane](float v, auto m) {
+        const float o = xshfl(v, decltype(m)::value);
+        return lane_in(lane_bit_mask(decltype(m)::value)) ? o - v : v + o;
+    };
     for (int i = lane; i < B; i += 64) {
         float x = 0.0f;
         if (i < dim) {
@@ -573,19 +582,24 @@ __device__ __forceinline__ void prepare_query(const float *__restrict__ query, c
             if (qv) qv[i] = v;
             x = v * signs[i];
         }
+        x = pair(x, std::integral_constant<int, 1>{});
+        x = pair(x, std::integral_constant<int, 2>{});
+        x = pair(x, std::integral_constant<int, 4>{});
+        x = pair(x, std::integral_constant<int, 8>{});
+        x = pair(x, std::integral_constant<int, 16>{});
+        x = pair(x, std::integral_constant<int, 32>{});
         rot[i] = x;
     }
-    lead_sync<NW>();
-    for (int len = 1; len < B; len <<= 1) {
-        for (int p = lane; p < (B >> 1); p += 64) {
-            const int blk = p / len, j = p - blk * len;
-            const int i1 = blk * (len << 1) + j, i2 = i1 + len;
+    for (int len = 64; len < B; len <<= 1) {
+#pragma unroll 4
+        for (int q = lane; q < (B >> 1); q += 64) {
+            const int i1 = ((q & ~(len - 1)) << 1) | (q & (len - 1)), i2 = i1 + len;
             const float u = rot[i1], v = rot[i2];
             rot[i1] = u + v;
             rot[i2] = u - v;
         }
-        lead_sync<NW>();
     }
+    lead_sync<NW>();
     float lo = FLT_MAX, hi = -FLT_MAX;
     for (int i = lane; i < B; i += 64) {
         lo = fminf(lo, rot[i]);
@@ -843,8 +857,10 @@ __device__ __forceinline__ float half_distance(const float *__restrict__ row, co
     float val = 0.0f;
     if (active) {
         if (use_ip) {
+#pragma unroll 8
             for (int i = nl; i < dim; i += 32) val = fmaf(qv[i], row[i], val);
         } else {
+#pragma unroll 8
             for (int i = nl; i < dim; i += 32) {
                 const float d = qv[i] - row[i];
                 val = fmaf(d, d, val);
