@@ -143,7 +143,7 @@ constexpr uint32_t kMsortPairs = 37;
 // slots are written to pbeam + 2).
 constexpr uint32_t kBeamPad = 4;
 
-// A team launch runs each query on two waves, or on four for wide vectors: the
+// A team launch runs each query on two waves or on four (team_waves): the
 // lead wave runs the search; the helpers take their share of every stage-II
 // round (visited tests, estimates and keep decisions of their tasks), of every
 // exact-distance batch, of every visited-table rebuild and, at beams over 256,
@@ -1891,7 +1891,7 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
 // the workgroup barriers mark the meeting points.
 template <int WT, int DPL, int DIM_T, int DEG_T, bool COUNT, bool PROF, bool BIG, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : (DIM_T > 0 && NW == 1 && !COUNT && !PROF && !BIG ? 6 : 5)))) void fg_search_kernel(SearchParams P) {
-    static_assert(NW == 1 || NW == 2 || (NW == 4 && WT == 0), "team form: two waves, four for wide vectors");
+    static_assert(NW == 1 || NW == 2 || (NW == 4 && DEG_T != 16), "team form: two waves or four");
     extern __shared__ __align__(16) unsigned char smem[];
     int qid = blockIdx.x;
     if (qid >= P.nq) return;
@@ -2760,19 +2760,45 @@ inline long long resident_groups(const void *kernel, int threads, uint32_t lds) 
 // form's two launches 6.7 ms, in the team form 5.94; 2,000 queries 1.75 and
 // 1.61; 3,000 queries at beam 256 0.66 and 0.635).  Where the second wave does
 // cost slots the one-wave form is faster (10,000 queries at beam 256: +19% in
-// the team form).  Four waves, for wide vectors (four_wave_kernel), when the
-// device holds the batch in that form too: there the stages that share out,
-// the estimates and exact distances, are most of an iteration (d 960, beam 384:
-// 1,000 queries 0.970 ms in two waves, 0.929 in four, 100 queries 0.763 and
-// 0.652; d 1536, beam 640: 64 queries 1.78 ms before and 1.18).
-// FLASHGANN_TEAM=0 / 1 forces the one-wave / a team form (tests run both).
+// the team form).
+//
+// Four waves (four_wave_kernel; the degree-16 geometry packs a round into two
+// sub-rounds and has none) where four_waves_pay says so and the device holds
+// the batch in that form: the shared stages shrink further, the lead wave's own
+// phases do not.  Two waves -> four:
+//   padded dimension 512 and more, whose estimates and exact distances are most
+//   of an iteration: d 960, beam 384, 1,000 queries 0.970 -> 0.929 ms, 100
+//   queries 0.763 -> 0.652; d 1536, beam 640, 64 queries 1.78 -> 1.18;
+//   d 200, us: one query at beam 64 109 -> 99, at 300 295 -> 267; 64 queries at
+//   beam 128 210 -> 192, at 1024 1,061 -> 900; 777 at 300 437 -> 417, but 1,200
+//   474 -> 484;
+//   d 128, us: one query at beam 128 119 -> 112; 64 queries at 256 280 -> 266,
+//   at 1024 921 -> 813; 1,200 at 128 226 -> 223, but 777 at 300 364 -> 368 and
+//   1,200 398 -> 422.
+// Above beam 256 every wave sorts the candidates, so a fuller device pays for
+// the copies: there three quarters of the resident batch at padded dimension
+// 256, half below it.  At beams up to 64 and padded dimension up to 128 the gain
+// is 1-5% (64 queries at d 128 129 -> 125 us) and two waves stay, the form
+// that fg_search_waves has always given for such searches.
+// FLASHGANN_TEAM=0 forces the one-wave form, 1 a team form, 2 or 4 that team
+// form (two where there are no four; tests run them).
+inline bool four_waves_pay(const SearchParams &P, long long resident) {
+    if (P.padded_dim <= 128 && P.beam <= 64) return false;
+    if (P.padded_dim <= 256 && P.pbeam > 256) resident = P.padded_dim > 128 ? resident * 3 / 4 : resident / 2;
+    return P.nq <= resident;
+}
+
 inline int team_waves(const SearchParams &P, const void *one_wave_kernel, const void *two_wave_kernel,
                       const void *four_wave_kernel) {
     if (!P.team) return 1;
     const char *e = std::getenv("FLASHGANN_TEAM");
-    if (e && e[0] == '0') return 1;
-    if (four_wave_kernel && P.nq <= resident_groups(four_wave_kernel, 256, P.lds.total_team)) return 4;
-    if (e && e[0] == '1') return 2;
+    const char want = e ? e[0] : 0;
+    if (want == '0') return 1;
+    if (four_wave_kernel && want == '4') return 4;
+    if (four_wave_kernel && want != '2' &&
+        four_waves_pay(P, resident_groups(four_wave_kernel, 256, P.lds.total_team)))
+        return 4;
+    if (want == '1' || want == '2' || want == '4') return 2;
     const long long team = resident_groups(two_wave_kernel, 128, P.lds.total_team);
     if (P.nq <= team) return 2;
     return 10 * team >= 9 * resident_groups(one_wave_kernel, 64, P.lds.total) ? 2 : 1;
@@ -2799,7 +2825,7 @@ void launch_geo_b(const SearchParams &P, hipStream_t stream, bool count, bool pr
     const void *one = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 1>);
     const void *two = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 2>);
     const void *four = nullptr;
-    if constexpr (WT == 0)
+    if constexpr (DEG_T != 16)
         four = reinterpret_cast<const void *>(&fg_search_kernel<WT, DPL, DIM_T, DEG_T, false, false, BIG, 4>);
     const int waves = one_wave ? 1 : team_waves(P, one, two, four);
     if (waves_only) {  // the form only, no launch
@@ -2807,7 +2833,7 @@ void launch_geo_b(const SearchParams &P, hipStream_t stream, bool count, bool pr
         if (resident) *resident = resident_groups(one, 64, P.lds.total);
         return;
     }
-    if constexpr (WT == 0) {
+    if constexpr (DEG_T != 16) {
         if (waves == 4) {
             launch_form<WT, DPL, DIM_T, DEG_T, BIG, 4>(P, stream, count, prof);
             return;

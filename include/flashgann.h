@@ -168,10 +168,11 @@ uint32_t fg_lds_bytes(uint32_t dim, uint32_t beam, uint32_t degree);
 /* Waves per query (1, 2 or 4) that a search of nq queries at this K and beam
  * launches on the current device: two, the kernel's team form, when a second
  * wave per query costs no query a slot (the device holds the whole batch in
- * the team form, or, at wide beams, as many queries in either form), four for
- * vectors of more than 256 dimensions when the device holds the batch in that
- * form;
- * FLASHGANN_TEAM=0/1 in the environment forces one form.  Results are
+ * the team form, or, at wide beams, as many queries in either form), four where
+ * the device holds the batch in that form and it measured faster (not for d 96,
+ * degree 16, nor at beams up to 64 below 129 dimensions, nor for a fuller
+ * device at beams over 256).  FLASHGANN_TEAM in the environment forces the
+ * one-wave form (0), a team form (1) or that team form (2, 4).  Results are
  * identical either way.
  * Negative FG_E* on invalid arguments.  No counterpart in the reference (one
  * warp-per-parent block shape). */

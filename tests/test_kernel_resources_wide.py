@@ -18,4 +18,4 @@ def test_padded_256_kernels_use_no_scratch(tmp_path):
     subprocess.run([HIPCC, *_flags(), "-DFG_SHAPE=7", "--cuda-device-only", "-S", "-o", str(out), src], check=True,
                    capture_output=True, timeout=900)
     sizes = [int(x) for x in re.findall(r"; ScratchSize: (\d+)", out.read_text())]
-    assert len(sizes) == 12 and not any(sizes), sizes
+    assert len(sizes) == 18 and not any(sizes), sizes
