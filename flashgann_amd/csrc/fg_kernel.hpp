@@ -253,7 +253,7 @@ struct SearchParams {
     int dup_free;
     int vec_ok;
     int runtime_geo;  // host only: run the runtime-geometry kernels
-    int team;         // host only: the team form (two waves per query) may run
+    int team;         // host only: the team form (two or four waves per query) may run
     uint32_t entry;
     int nq;
     // Sliced search (one-wave form): a slice that suspends

@@ -13,7 +13,7 @@
 //     same compare-exchange sequence is replayed on the wave (two 32-lane
 //     halves, or 1-2 positions per lane) and ties resolve identically;
 //   * RaBitQ scores come from the matrix unit: the quantized query's levels
-//     as rows of base-4 digits times the code bits, both as 4-bit floats
+//     as rows of base-5 digits times the code bits, both as 4-bit floats
 //     (raw_mfma), corrected for the reference's uint8 LUT wrap, instead of
 //     per-nibble LUT gathers;
 //   * exact distances keep the reference's per-lane accumulation order and
