@@ -561,8 +561,12 @@ def _encode_rows_gpu(x: torch.Tensor, nbrs: torch.Tensor, signs: np.ndarray, lay
     staging blocks of at most `stage_bytes` (one row if that is more), and
     while one is being filled the host copies the other into the result."""
     from . import _lib
-    n, degree = nbrs.shape
-    x, nbrs = x.contiguous(), nbrs.contiguous()
+    n, degree = x.shape[0], nbrs.shape[1]
+    # the kernel reads one graph row and one vector per node, and a neighbour's
+    # vector by its id: every one of them must be there
+    if nbrs.shape[0] < n:
+        raise RuntimeError(f"the graph has {nbrs.shape[0]} rows for {n} points")
+    x, nbrs = x.contiguous(), nbrs[:n].contiguous()
     if int(nbrs.max()) >= n:
         raise IndexError(f"neighbour id out of range for {n} points")
     sg = torch.as_tensor(np.ascontiguousarray(signs, dtype=np.float32), device=x.device)

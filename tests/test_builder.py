@@ -5,6 +5,7 @@ from __future__ import annotations
 import ctypes as C
 
 import numpy as np
+import pytest
 
 from conftest import small_index
 from oracle import oracle as O
@@ -269,3 +270,32 @@ def test_connected_graph_keeps_rng_edges_and_reaches_every_node():
         ids, _ = O.OracleIndex.from_codebook(cb).search(q, 10, 64)
         rec.append(O.recall(ids, gt, 10))
     assert rec[0] < 0.1 and rec[1] > 0.4 and rec[1] > 5 * rec[0], rec
+
+
+@pytest.mark.parametrize("extra", [-10, -1, 1, 10])
+def test_graph_of_another_length(extra):
+    """A graph with more rows than there are vectors encodes the vectors' rows;
+    one with fewer is refused.  The device path bounds ids and rows by the
+    vectors as well, before it touches the device (its tensors are on the CPU
+    here): its kernel would read past them."""
+    import torch
+    from flashgann_amd import builder, datasets
+    from flashgann_amd.codebook import Layout, padded_dim_for
+    n, dim, degree = 50, 40, 4
+    rng = np.random.default_rng(2)
+    base = rng.integers(0, 50, size=(n, dim)).astype(np.float32)
+    nbrs = rng.integers(0, min(n, n + extra), size=(n + extra, degree))
+    signs = datasets.signs_for(padded_dim_for(dim))
+    x, lay = torch.as_tensor(base), Layout.make(dim, degree)
+    if extra < 0:
+        with pytest.raises(RuntimeError):
+            builder.codebook_from_graph(base, nbrs, signs, entry=0)
+        with pytest.raises(RuntimeError, match="rows for 50 points"):
+            builder._encode_rows_gpu(x, torch.as_tensor(nbrs), signs, lay, False)
+        return
+    a = builder.codebook_from_graph(base, nbrs, signs, entry=0)
+    b = builder.codebook_from_graph(base, nbrs[:n], signs, entry=0)
+    assert a.npoints == n and np.array_equal(a.rows.view(np.uint32), b.rows.view(np.uint32))
+    nbrs[3, 1] = n  # no such vector, though the graph has that many rows
+    with pytest.raises(IndexError):
+        builder._encode_rows_gpu(x, torch.as_tensor(nbrs), signs, lay, False)

@@ -119,3 +119,21 @@ def test_gpu_encode_kernel_equals_cpu_encoding(gpu_available, dim, degree, use_i
     nb[0, 0] = n
     with pytest.raises(IndexError):
         builder._encode_rows_gpu(x, nb, signs, a.layout, use_ip)
+
+
+def test_gpu_encoding_ignores_graph_rows_past_the_vectors(gpu_available):
+    """A graph of more rows than vectors encodes the vectors' rows, as on the
+    CPU, whatever ids the further rows hold; a shorter one is refused."""
+    from flashgann_amd import builder, datasets
+    from flashgann_amd.codebook import padded_dim_for
+    n, dim, degree = 50, 40, 4
+    rng = np.random.default_rng(2)
+    base = rng.integers(0, 50, size=(n, dim)).astype(np.float32)
+    nbrs = rng.integers(0, n, size=(n + 10, degree))
+    nbrs[n:] = n + 3
+    signs = datasets.signs_for(padded_dim_for(dim))
+    a = builder.codebook_from_graph(base, nbrs, signs, device="cpu", entry=0)
+    b = builder.codebook_from_graph(base, nbrs, signs, device="cuda", entry=0)
+    assert np.array_equal(a.rows.view(np.uint32), b.rows.view(np.uint32))
+    with pytest.raises(RuntimeError):
+        builder.codebook_from_graph(base, nbrs[:n - 1], signs, device="cuda", entry=0)
