@@ -2780,8 +2780,8 @@ inline long long resident_groups(const void *kernel, int threads, uint32_t lds) 
 // 256, half below it.  At beams up to 64 and padded dimension up to 128 the gain
 // is 1-5% (64 queries at d 128 129 -> 125 us) and two waves stay, the form
 // that fg_search_waves has always given for such searches.
-// FLASHGANN_TEAM=0 forces the one-wave form, 1 a team form, 2 or 4 that team
-// form (two where there are no four; tests run them).
+// FLASHGANN_TEAM=0 forces the one-wave form, 1 or 2 two waves, 4 four (two
+// where there are no four); tests run them all.
 inline bool four_waves_pay(const SearchParams &P, long long resident) {
     if (P.padded_dim <= 128 && P.beam <= 64) return false;
     if (P.padded_dim <= 256 && P.pbeam > 256) resident = P.padded_dim > 128 ? resident * 3 / 4 : resident / 2;
@@ -2794,11 +2794,9 @@ inline int team_waves(const SearchParams &P, const void *one_wave_kernel, const 
     const char *e = std::getenv("FLASHGANN_TEAM");
     const char want = e ? e[0] : 0;
     if (want == '0') return 1;
-    if (four_wave_kernel && want == '4') return 4;
-    if (four_wave_kernel && want != '2' &&
-        four_waves_pay(P, resident_groups(four_wave_kernel, 256, P.lds.total_team)))
-        return 4;
-    if (want == '1' || want == '2' || want == '4') return 2;
+    if (want == '1' || want == '2') return 2;
+    if (want == '4') return four_wave_kernel ? 4 : 2;
+    if (four_wave_kernel && four_waves_pay(P, resident_groups(four_wave_kernel, 256, P.lds.total_team))) return 4;
     const long long team = resident_groups(two_wave_kernel, 128, P.lds.total_team);
     if (P.nq <= team) return 2;
     return 10 * team >= 9 * resident_groups(one_wave_kernel, 64, P.lds.total) ? 2 : 1;

@@ -171,8 +171,8 @@ uint32_t fg_lds_bytes(uint32_t dim, uint32_t beam, uint32_t degree);
  * the team form, or, at wide beams, as many queries in either form), four where
  * the device holds the batch in that form and it measured faster (not for d 96,
  * degree 16, nor at beams up to 64 below 129 dimensions, nor for a fuller
- * device at beams over 256).  FLASHGANN_TEAM in the environment forces the
- * one-wave form (0), a team form (1) or that team form (2, 4).  Results are
+ * device at beams over 256).  FLASHGANN_TEAM in the environment forces one
+ * wave (0), two (1 or 2) or four (4; two at d 96, degree 16).  Results are
  * identical either way.
  * Negative FG_E* on invalid arguments.  No counterpart in the reference (one
  * warp-per-parent block shape). */

@@ -38,12 +38,14 @@ def small_index(n=3000, nq=24, dim=128, comps=16, degree=32, kind="int", use_ip=
     return cb, q, base
 
 
-@pytest.fixture(params=["one-wave", "team"])
+@pytest.fixture(params=["one-wave", "team", "four-wave"])
 def search_form(request, monkeypatch):
     """Runs a GPU test once with each form of the search kernel: one wave
-    per query, and the team form (two waves per query) that small launches
-    use.  FLASHGANN_TEAM is read at every launch."""
-    monkeypatch.setenv("FLASHGANN_TEAM", "0" if request.param == "one-wave" else "1")
+    per query, the team form of two that small and half-full launches use, and
+    the team form of four that smaller ones use (two again for the fixed
+    geometry of degree 16, which has no four).  FLASHGANN_TEAM is read at
+    every launch."""
+    monkeypatch.setenv("FLASHGANN_TEAM", {"one-wave": "0", "team": "1", "four-wave": "4"}[request.param])
     return request.param
 
 

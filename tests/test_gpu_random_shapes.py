@@ -1,7 +1,7 @@
 """GPU parity over seeded random search shapes: dimension (33-1536, so
 every shape class: fixed and runtime geometry, padded dimensions 64-2048),
 degree (1-96, one to three tiles), K, beam (1-1024, both merge families),
-metric, data family, kernel form (one wave / team) and schedule (one launch /
+metric, data family, kernel form (one wave, or the team form of two or four) and schedule (one launch /
 two).  Each case builds a small codebook on the CPU and requires the
 kernel's ids and per-query work counters to equal the CPU oracle's."""
 from __future__ import annotations
@@ -31,11 +31,20 @@ def _case(seed):
 
 @pytest.mark.parametrize("seed", range(48))
 def test_random_shape_matches_oracle(gpu_available, monkeypatch, seed):
+    _check(monkeypatch, seed)
+
+
+@pytest.mark.parametrize("seed", range(48, 72))
+def test_random_shape_four_waves(gpu_available, monkeypatch, seed):
+    _check(monkeypatch, seed, team="4")
+
+
+def _check(monkeypatch, seed, team=None):
     from flashgann_amd import Index
     from oracle import oracle as O
     c = _case(seed)
     print(f"random shape {seed}: {c}", flush=True)
-    monkeypatch.setenv("FLASHGANN_TEAM", "1" if c["team"] else "0")
+    monkeypatch.setenv("FLASHGANN_TEAM", team or ("1" if c["team"] else "0"))
     monkeypatch.setenv("FLASHGANN_SLICE", "1" if c["slice"] else "0")
     if c["runtime"]:
         monkeypatch.setenv("FG_FORCE_RUNTIME_GEOMETRY", "1")
