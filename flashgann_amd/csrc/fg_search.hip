@@ -601,6 +601,8 @@ struct fg_index {
     hipEvent_t serve_done[kMaxServeStreams] = {};
     hipEvent_t serve_start = nullptr;
     int serve_count = 0;
+    // whether a fg_search_stream call made its one launch on the caller's stream
+    bool on_caller = false;
 };
 
 namespace {
@@ -1092,6 +1094,15 @@ void fg_index_destroy(fg_index *ix) {
     // two-launch search) end before any of its memory is released
     if (ix->slice_done) (void)hipEventSynchronize(ix->slice_done);
     for (int i = 0; i < ix->serve_count; ++i) (void)hipStreamSynchronize(ix->serve[i]);
+    // fg_search_stream calls of one launch ran on streams of the caller's, any
+    // number of them (hipFree below waits for the device as well)
+    if (ix->on_caller) {
+        int cur = ix->device;
+        (void)hipGetDevice(&cur);
+        (void)hipSetDevice(ix->device);
+        (void)hipDeviceSynchronize();
+        (void)hipSetDevice(cur);
+    }
     if (ix->d_rows) (void)hipFree(ix->d_rows);
     if (ix->d_signs) (void)hipFree(ix->d_signs);
     if (ix->d_q) (void)hipFree(ix->d_q);
@@ -1162,6 +1173,7 @@ int fg_search_stream(fg_index *ix, const float *d_queries, uint32_t nq, uint32_t
         P.results = d_results;
         P.counters = nullptr;
         P.phase = nullptr;
+        ix->on_caller = true;
         return launch(ix, P, caller, true);
     }
     while (ix->serve_count < static_cast<int>(nstreams)) {

@@ -302,6 +302,33 @@ def test_search_stream_matches_single_launch(gpu_available, batch, nstreams):
     assert np.array_equal(got.numpy().view(np.uint32), oids)
 
 
+@pytest.mark.parametrize("nq,batch,nstreams", [(24, 5, 2), (300, 300, 1), (7000, 1000, 3), (40000, 1000, 2)])
+def test_index_closed_after_a_stream_call(gpu_available, nq, batch, nstreams):
+    """The index waits for fg_search_stream's searches before it is released,
+    on the caller's stream (one launch) as on its own (several): closed right
+    after the call, behind other work on that stream, the ids are whole."""
+    import torch
+    from flashgann_amd import Index
+    from oracle import oracle as O
+    cb, q, _ = small_index(n=3000, nq=300)
+    ix = Index.from_codebook(cb)
+    dq = torch.as_tensor(q, device="cuda").repeat(-(-nq // q.shape[0]), 1)[:nq].contiguous()
+    out = torch.full((nq, 10), -1, dtype=torch.int32, device="cuda")
+    work = torch.ones((4096, 4096), device="cuda")
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        for _ in range(8):
+            work = (work @ work) * 1e-4
+    ix.search_stream(dq.data_ptr(), nq, 10, 128, out.data_ptr(), batch, nstreams, s.cuda_stream)
+    ix.close()
+    if nq <= 16384:  # one launch, on s: it has ended (of several, s only waits for the index's streams)
+        assert s.query()
+    got = out.cpu().numpy().view(np.uint32)
+    rids, _ = O.OracleIndex.from_codebook(cb).search(q, 10, 128)
+    assert np.array_equal(got, rids[np.arange(nq) % q.shape[0]])
+
+
 @pytest.mark.parametrize("dim,degree,kind", [(128, 32, "int"), (96, 32, "unit"), (96, 16, "unit")])
 def test_fixed_geometry_matches_runtime_geometry(gpu_available, dim, degree, kind, monkeypatch):
     """The kernels specialised for the benchmark shapes (32-bit row offsets,
