@@ -281,9 +281,9 @@ def test_cli_end_to_end(gpu_available, tmp_path, cli_name):
 
 @pytest.mark.parametrize("batch,nstreams", [(5, 1), (5, 2), (7, 3), (24, 2), (100, 4)])
 def test_search_stream_matches_single_launch(gpu_available, batch, nstreams):
-    """fg_search_stream (batches on internal streams) returns, in query order,
-    the ids of one fg_search_device launch over the same queries, and the
-    caller's stream sees them complete."""
+    """fg_search_stream (batches that together fit one launch, on the caller's
+    stream) returns, in query order, the ids of one fg_search_device launch over
+    the same queries, and the caller's stream sees them complete."""
     import torch
     from flashgann_amd import Index
     cb, q, _ = small_index()
@@ -300,6 +300,39 @@ def test_search_stream_matches_single_launch(gpu_available, batch, nstreams):
     from oracle import oracle as O
     oids, _ = O.OracleIndex.from_codebook(cb).search(q, 100, 128)
     assert np.array_equal(got.numpy().view(np.uint32), oids)
+
+
+@pytest.mark.parametrize("nq,batch,nstreams", [(16001, 1000, 2), (40000, 1000, 2), (40001, 9000, 4), (33000, 1, 1),
+                                               (40000, 20000, 2), (50001, 16384, 8), (20000, 16383, 3)])
+def test_search_stream_several_launches(gpu_available, nq, batch, nstreams):
+    """fg_search_stream over more queries than a launch takes (16,384, rounded
+    down to whole batches; one batch where that is larger): the internal
+    streams, each launch's queries and results, a short last launch.  The
+    queries are written and the results read on the caller's stream, right
+    before and after, and a second call reuses the streams.  16,001 queries in
+    batches of 1,000 are one launch of 16,000 and one of a single query."""
+    import torch
+    from flashgann_amd import Index
+    from oracle import oracle as O
+    cb, q, _ = small_index(n=3000, nq=300)
+    ix = Index.from_codebook(cb)
+    src = torch.as_tensor(q, device="cuda").repeat(-(-nq // q.shape[0]), 1)[:nq].contiguous()
+    rids, _ = O.OracleIndex.from_codebook(cb).search(q, 10, 128)
+    want = rids[np.arange(nq) % q.shape[0]]
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        for _ in range(2):
+            dq = torch.zeros_like(src)
+            out = torch.full((nq, 10), -1, dtype=torch.int32, device="cuda")
+            work = torch.ones((4096, 4096), device="cuda")
+            for _ in range(4):
+                work = (work @ work) * 1e-4
+            dq.copy_(src)  # behind the products
+            ix.search_stream(dq.data_ptr(), nq, 10, 128, out.data_ptr(), batch, nstreams, s.cuda_stream)
+            got = out.cpu().numpy().view(np.uint32)
+            assert np.array_equal(got, want)
+    ix.close()
 
 
 @pytest.mark.parametrize("nq,batch,nstreams", [(24, 5, 2), (300, 300, 1), (7000, 1000, 3), (40000, 1000, 2)])
