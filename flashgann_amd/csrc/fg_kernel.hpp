@@ -627,9 +627,9 @@ __device__ __forceinline__ void prepare_query(const float *__restrict__ query, c
         // nl >> 2.  The 4-bit floats of 0 .. 3 times 2, 1, 1/2, as nibbles:
         const uint32_t r = static_cast<uint32_t>(nl) & 3u;
         const uint32_t table = r == 1u ? 0x5420u : r == 2u ? 0x3210u : 0x7640u;
-        // (a spread too small for fp32, whose inverse overflows, gives levels
-        // past 64, which the width of such a query makes immaterial)
-        int rest = static_cast<int>(min(q, 64u));
+        // (a spread too small for fp32, whose inverse overflows, gives every
+        // level but the lowest as 2^32 - 1: six bits of q - 1 remain, level 63)
+        int rest = q != 0u ? static_cast<int>(((q - 1u) & 63u) + 1u) : 0;
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             const int up = (rest + 2) / 5, digit = t < 2 ? rest - 5 * up : rest;

@@ -505,17 +505,21 @@ __global__ __launch_bounds__(64) void fg_score_kernel(ScoreParams S) {
     const uint32_t *code = reinterpret_cast<const uint32_t *>(prow + S.code_offset) + static_cast<uint64_t>(slot) * W;
     const float *f = prow + S.factor_offset;
     const float tx = f[slot], fdq = f[S.deg + slot], fvq = f[2 * S.deg + slot];
-    // the levels summed chunk by chunk, each chunk's sum taken mod 256 as the
-    // reference's uint8 LUT entry is (utils.cuh:909-917, 976-980), the halves
-    // splitting the words (theta == 1 layout); and the search kernel's own
-    // routines on all words (theta > 1 layout): the integer sums must agree.
+    // the levels summed chunk by chunk, less 256 where the reference's uint8 LUT
+    // entry wraps (utils.cuh:909-917, 976-980), the halves splitting the words
+    // (theta == 1 layout); and the search kernel's own routines on all words
+    // (theta > 1 layout): the integer sums must agree.
+    const uint32_t *wrap = reinterpret_cast<const uint32_t *>(prep + prep_wrap_off(static_cast<uint32_t>(W)));
     int32_t part = 0;
     for (int wd = h * (W >> 1); wd < (h + 1) * (W >> 1); ++wd) {
-        const uint32_t c = code[wd];
+        const uint32_t c = code[wd], x = c & wrap[wd];
         for (int k = 0; k < 8; ++k) {
-            uint32_t sum = 0;
-            for (int d = 0; d < 4; ++d) sum += ((c >> (4 * k + 3 - d)) & 1u) * levels[32 * wd + 4 * k + d];
-            part += static_cast<int32_t>(sum & 255u);
+            for (int d = 0; d < 4; ++d) {
+                // (255 stands for 2^32 - 1, which prepare_query takes as 63)
+                const int32_t level = levels[32 * wd + 4 * k + d];
+                part += ((c >> (4 * k + 3 - d)) & 1u) != 0u ? (level == 255 ? 63 : level) : 0;
+            }
+            part -= ((x >> (4 * k)) & 15u) == 15u ? 256 : 0;
         }
     }
     const float raw_split = static_cast<float>(add32i(part));

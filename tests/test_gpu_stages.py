@@ -151,3 +151,38 @@ def test_zero_level_query_scores_and_search(gpu_available, kind, dim, n):
     assert np.array_equal(ids, rids)
     assert np.array_equal(cnt, rcnt.view(np.uint32).reshape(-1, 6))
     ix.close()
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256, 512, 2048])
+def test_tiny_spread_query_scores(gpu_available, dim):
+    """A query so small that the inverse of its level width overflows: every
+    level but the lowest saturates (dumped as 255) and counts as 63, a full
+    chunk that holds one less 256, in both estimators.  Edge factors as large
+    as the width is small make the sums visible; the expected estimate is the
+    formula in float64 (each product of two float32 is exact there)."""
+    from flashgann_amd import Index
+    cb, _, _ = small_index(n=700, nq=4, dim=dim, comps=4)
+    lay = cb.layout
+    rows = cb.rows.copy()
+    rows[:, :dim] = 0.0
+    fac = rows[:, lay.factor_offset:lay.neighbor_offset].reshape(-1, 3, lay.degree)
+    fac[:, 0], fac[:, 1], fac[:, 2] = 0.0, 1e37, 0.0
+    rng = np.random.default_rng(4)
+    q = (rng.integers(-20, 20, size=(3, dim)) * 1e-41).astype(np.float32)
+    ix = Index.from_rows(rows, cb.signs, dim, lay.degree, 0, 0)
+    _, lv, lhw, sq = ix.query_prepare(q)
+    assert (np.unique(lv) == (0, 255)).all() and (lhw[:, 2] > 0).all()
+    m = 150
+    qi = rng.integers(0, 3, m).astype(np.uint32)
+    pa = rng.integers(0, rows.shape[0], m).astype(np.uint32)
+    sl = rng.integers(0, lay.degree, m).astype(np.uint32)
+    el, es, _ = ix.score_edges(q, qi, pa, sl)
+    ix.close()
+    codes = cb.codes()
+    for t in range(m):
+        level = np.where(lv[qi[t]] == 255, 63, 0).reshape(-1, 4)
+        nib = np.stack([codes[pa[t], sl[t]] & 15, codes[pa[t], sl[t]] >> 4], 1).reshape(-1)
+        bits = (nib[:, None] >> np.array([3, 2, 1, 0])) & 1
+        raw = int((level * bits).sum()) - 256 * int(((nib == 15) & (level != 0).any(1)).sum())
+        want = np.float32(np.float64(np.float32(np.float32(1e37) * lhw[qi[t], 2])) * (2 * raw - int(sq[qi[t]])))
+        assert el[t] == want and es[t] == want, (t, el[t], es[t], want)
