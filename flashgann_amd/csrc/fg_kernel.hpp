@@ -166,6 +166,13 @@ constexpr uint32_t kTeamBytes = 192;
 static_assert(sizeof(TeamBlock) <= kTeamBytes, "team block");
 constexpr uint32_t kProfBytes = 16u * 8u;
 
+// The index in a wave's list of kept children that names the beam's pad entry
+// pbeam + 2, where a lane with nothing to list writes.  A helper's list lies
+// past the beam, so the index is negative there, and signed.
+__host__ __device__ __forceinline__ int list_spare(const uint32_t *list, const uint2 *bp, int pbeam) {
+    return static_cast<int>(reinterpret_cast<const uint32_t *>(bp + pbeam + 2) - list);
+}
+
 // The lead wave's way out of the search loop in the team form: it tells the
 // helper to stop at their meeting point (the helper then leaves too).
 template <int NW>
@@ -2552,9 +2559,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 // lane's place is the running total plus its rank among the
                 // kept lanes of the wave.  A lane with nothing to list, and one
                 // past the 32nd place, writes the beam's pad entry that takes
-                // the merge's unused slots: no branch.  The helper's tasks
-                // follow the lead wave's: it lists its own, and the lead wave
-                // reads both lists.
+                // the merge's unused slots: no branch.  The helpers' tasks
+                // follow the lead wave's: each lists its own, and the lead wave
+                // reads all lists.
                 uint32_t total = 0;
                 {
                     constexpr int kHelpers = NW > 1 ? NW - 1 : 1;
@@ -2562,13 +2569,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                     static_assert(kHelpers * kRoom <= 32u, "team lists");
                     uint32_t *list = lead ? alist : tb->list + kRoom * static_cast<uint32_t>(wv - 1);
                     const uint32_t room = lead ? 32u : kRoom;
-                    const uint32_t spare =
-                        static_cast<uint32_t>(reinterpret_cast<uint32_t *>(bp + pbeam + 2) - list);
+                    const int spare = list_spare(list, bp, pbeam);
 #pragma unroll
                     for (int sr = 0; sr < SRN; ++sr) {
                         const uint32_t e = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(klm[sr] >> 32),
                                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(klm[sr]), total));
-                        list[(lane_in(klm[sr]) & (e < room)) ? e : spare] = cid[sr];
+                        list[(lane_in(klm[sr]) & (e < room)) ? static_cast<int>(e) : spare] = cid[sr];
                         total += static_cast<uint32_t>(__popcll(klm[sr]));
                     }
                 }
