@@ -665,6 +665,7 @@ __device__ __forceinline__ void prepare_query(const float *__restrict__ query, c
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
 // Where a lane reads its part of the matrix operand that holds the prepared
 // query (raw_mfma): the address of code word 0's row, and the step from word
@@ -803,7 +804,10 @@ __device__ __forceinline__ void raw_span(const uint32_t *const (&code)[NB], cons
             if (vec_ok) {
 #pragma unroll
                 for (int j = 0; j < NWD / 4; ++j) {
-                    const uint4 v = reinterpret_cast<const uint4 *>(code[b] + w0)[j];
+                    // (a vector type: a struct's load is four words to the compiler,
+                    // which then shared its words with the branch below and
+                    // loaded all sixteen one by one)
+                    const v4u v = reinterpret_cast<const v4u *>(code[b] + w0)[j];
                     c[b][4 * j] = v.x; c[b][4 * j + 1] = v.y; c[b][4 * j + 2] = v.z; c[b][4 * j + 3] = v.w;
                 }
             } else {
