@@ -66,6 +66,17 @@ __host__ __device__ inline uint32_t effective_sort_beam(uint32_t beam) {
 __host__ __device__ inline int clamp_i(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 __host__ __device__ inline float clamp_f(float v, float lo, float hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
+// task * tile_inverse(tiles) >> 16 is task / tiles for every task of a search
+// width of parents and rows of up to kMaxDegree / 32 tiles.
+__host__ __device__ constexpr uint32_t tile_inverse(uint32_t tiles) { return tiles > 1 ? 65536u / tiles + 1u : 65536u; }
+constexpr bool tile_inverse_exact() {
+    for (uint32_t tiles = 1; tiles <= static_cast<uint32_t>(kMaxDegree) / 32u; ++tiles)
+        for (uint32_t task = 0; task < static_cast<uint32_t>(kSearchWidth) * tiles; ++task)
+            if ((task * tile_inverse(tiles)) >> 16 != task / tiles) return false;
+    return true;
+}
+static_assert(tile_inverse_exact(), "tile_inverse");
+
 // utils.cuh:104-117
 __host__ __device__ inline int keep_count_per_parent(uint32_t max_degree, float rho) {
     float kf = 1.0f - rho;
@@ -1890,7 +1901,8 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
     } while (0)
 
 // One wave per workgroup; the register budget targets 5 waves per SIMD
-// (<= 96 VGPRs), 6 (<= 80) for the fixed geometries at beams up to 256, where
+// (<= 96 VGPRs), 6 (<= 80) for the fixed geometries at beams up to 256 and the
+// runtime ones that kTwoKeys and kParentAgain name, where
 // LDS allows 25 workgroups a CU (against 5 waves: d 128, beam 256, 40,000
 // queries 4.61 -> 4.44 ms, 5,500 0.933 -> 0.886, 10,000, whose time is its
 // longest queries', the same; d 96, 10,000 queries 1.004 -> 0.977).  Padded
@@ -1901,7 +1913,7 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
 // exact distances; `lead_sync` orders the lead wave's own LDS accesses and
 // the workgroup barriers mark the meeting points.
 template <int WT, int DPL, int DIM_T, int DEG_T, bool COUNT, bool PROF, bool BIG, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : (DIM_T > 0 && NW == 1 && !COUNT && !PROF && !BIG ? 6 : 5)))) void fg_search_kernel(SearchParams P) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : (NW == 1 && !COUNT && !PROF && (!BIG || WT == 2) && (DIM_T > 0 || DPL < 4) ? 6 : 5)))) void fg_search_kernel(SearchParams P) {
     static_assert(NW == 1 || NW == 2 || (NW == 4 && DEG_T != 16), "team form: two waves or four");
     extern __shared__ __align__(16) unsigned char smem[];
     int qid = blockIdx.x;
@@ -1934,6 +1946,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
     // fixed-size regions at compile-time offsets for the specialised shapes
     // (the same layout function the host sizes the launch with)
     constexpr bool kFixedGeo = Geo<DIM_T, DEG_T>::kFixed;
+    // The one-wave runtime geometries of padded dimension 64, and of 128 with
+    // d <= 96, hold the sixth wave per SIMD (80 registers) by two measures: at 64
+    // the visited tests of a round read two keys' buckets at a time, at 128 a
+    // task's parent is computed again where its distance is read.  With 81 and
+    // 91 registers a CU held 20 queries, and a batch of more than 5,120 fell into
+    // a second round of them: 6,000 queries at beam 128, degree 32: d 50 475 ->
+    // 383 us (417 before the branch-free tests took the registers), d 80 487 ->
+    // 409 (431).  Batches that fit either way: d 50 the same, d 80 3% slower, and
+    // with two tiles a row (d 66, degree 48, beam 256) 10,000 queries 7%.
+    constexpr bool kTwoKeys = NW == 1 && DIM_T == 0 && WT == 2;
+    constexpr bool kParentAgain = NW == 1 && !BIG && DIM_T == 0 && WT == 4 && DPL < 4;
     constexpr LdsLayout kL = lds_layout(DIM_T, Geo<DIM_T, DEG_T>::kB, 0, 0);
     const uint32_t msort_off = kFixedGeo ? kL.msort_off : P.lds.msort_off;
     const uint32_t scratch_off = kFixedGeo ? kL.scratch_off : P.lds.scratch_off;
@@ -2374,6 +2397,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             constexpr int G = DEG_T == 16 ? 16 : 32;
             constexpr int TPW = 64 / G;
             const int grp = lane / G, nlg = lane % G;
+            const uint32_t tile_inv = tile_inverse(static_cast<uint32_t>(tiles));
             for (int rbase = 0; rbase < tasks; rbase += kSearchWidth) {
                 constexpr int SR = kSearchWidth / TPW;  // sub-rounds of TPW tasks
                 // this wave's sub-rounds: all of them, or in the team form
@@ -2454,7 +2478,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 // (b) visited test against the table as it stood at the round's start
 #pragma unroll
                 for (int sr = 0; sr < SRN; ++sr) val[sr] = cid[sr] != kMaxIndex && cid[sr] < np32;
-                hash_contains_n<SRN>(H, nbk, cid, val);
+                if constexpr (kTwoKeys) {
+                    static_assert(SRN == 4 || !kTwoKeys, "pairs of keys");
+                    uint32_t k0[2] = {cid[0], cid[1]}, k1[2] = {cid[2], cid[3]};
+                    bool v0[2] = {val[0], val[1]}, v1[2] = {val[2], val[3]};
+                    hash_contains_n<2>(H, nbk, k0, v0);
+                    asm volatile("" ::: "memory");
+                    hash_contains_n<2>(H, nbk, k1, v1);
+                    val[0] = v0[0]; val[1] = v0[1]; val[2] = v1[0]; val[3] = v1[1];
+                } else {
+                    hash_contains_n<SRN>(H, nbk, cid, val);
+                }
                 // (c) which tasks need estimates.  From here on predicates are
                 // lane masks taken straight from compares, and each task works
                 // on its own bits of them with scalar instructions, beside the
@@ -2522,8 +2556,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                 for (int sr = 0; sr < SRN; ++sr) {
                     // computed on every lane (most need it); a lane whose task
                     // needs no estimates is kept by its mask alone
+                    int pidx = pix[sr];
+                    if constexpr (kParentAgain) {
+                        // (a task past the last reads some entry of pdist; its
+                        // lanes are not valid)
+                        const uint32_t task = static_cast<uint32_t>(rbase + TPW * sr + (lane_id_opaque() >> 5));
+                        pidx = static_cast<int>(min(__umul24(task, tile_inv) >> 16, static_cast<uint32_t>(kSearchWidth - 1)));
+                    }
                     const float e = estimate_formula(raw[sr], sumq_f, qwidth, qlow, tx[sr], fdq[sr], fvq[sr],
-                                                     pdist[pix[sr]]);
+                                                     pdist[pidx]);
                     est[sr] = tx[sr] != FLT_MAX ? e : FLT_MAX;
                     // a scored child with a non-finite estimate is dropped
                     // (finiteness as an integer compare on opaque bits, which
