@@ -234,21 +234,38 @@ __host__ __device__ constexpr LdsLayout lds_layout(uint32_t dim, uint32_t padded
 // (measured: 7,632-byte workgroups fit 21 to a CU, 7,760-byte ones 18).
 constexpr uint32_t kLdsGranule = 1280;
 
-// The visited table a search uses: the roomiest table (at most 90% worst-case
-// load) that fits in as many LDS granules as the smallest one needs, so the
-// table never costs a workgroup per CU (beam 384: 21 instead of 18 per CU,
-// beam 512: 18 instead of 16, beam 1024: 10 instead of 9) and keeps its
-// slack where that is free (beam 256).
+// Workgroups that a CU's 160 KB of LDS holds.
+__host__ __device__ constexpr uint32_t lds_groups(uint32_t bytes) {
+    return 160u * 1024u / ((bytes + kLdsGranule - 1u) / kLdsGranule * kLdsGranule);
+}
+
+// The visited table of a launch larger than the device holds at once: the
+// roomiest (at most 90% worst-case load) that leaves a CU as many queries as the
+// smallest table does, in the one-wave form and in the team form of two, as
+// far as registers let it hold them: at most 32 and 16 up to padded dimension
+// 128 (8 waves per SIMD), 16 and 10 at 256, 11 and 6 above (3 waves per SIMD).
+// At d 128: beam 384 21 queries a CU, which the roomiest table would make 18,
+// beam 512 18 instead of 16, beam 1024 10 instead of 9.  Where registers or a
+// whole number of workgroups leave LDS free the table keeps its slack: near
+// full, lookups walk on.  On small sets, whose searches fill the table, at
+// beam 1024 and 98% against 90%, nine queries a CU either way: d 600, one query
+// 2.72 -> 1.52 ms, 10,000 29.6 -> 17.5; d 960, 10,000 34.3 -> 26.7.  Above
+// padded dimension 256 eleven queries a CU with slack beat twelve without
+// (d 400, degree 16, beam 777, 4,000 queries 4.33 ms at 99%, 3.75 at 90%).
 __host__ __device__ inline uint32_t visited_buckets(uint32_t dim, uint32_t padded_dim, uint32_t pbeam, uint32_t beam,
                                                     uint32_t degree) {
     const uint32_t lo = visited_buckets_min(beam, degree);
-    const uint32_t total = lds_layout(dim, padded_dim, pbeam, lo).total;
-    uint32_t cap = (total + kLdsGranule - 1u) / kLdsGranule * kLdsGranule;
-    // (room for the team form's block where it fits in the same granules: at
-    // beam 1024 the team form then holds as many queries as the one-wave form)
-    if (total + kTeamBytes <= cap) cap -= kTeamBytes;
+    const uint32_t most1 = padded_dim <= 128u ? 32u : padded_dim == 256u ? 16u : 11u;
+    const uint32_t most2 = padded_dim <= 128u ? 16u : padded_dim == 256u ? 10u : 6u;
+    const auto held = [&](uint32_t b, uint32_t &one, uint32_t &two) {
+        const LdsLayout L = lds_layout(dim, padded_dim, pbeam, b);
+        one = lds_groups(L.total) < most1 ? lds_groups(L.total) : most1;
+        two = lds_groups(L.total_team) < most2 ? lds_groups(L.total_team) : most2;
+    };
+    uint32_t one0, two0, one, two;
+    held(lo, one0, two0);
     uint32_t b = visited_buckets_roomy(beam, degree);
-    while (b > lo && lds_layout(dim, padded_dim, pbeam, b).total > cap) --b;
+    for (held(b, one, two); b > lo && (one < one0 || two < two0); held(b, one, two)) --b;
     return b;
 }
 
@@ -2853,8 +2870,27 @@ inline int team_waves(const SearchParams &P, const void *one_wave_kernel, const 
     return 10 * team >= 9 * resident_groups(one_wave_kernel, 64, P.lds.total) ? 2 : 1;
 }
 
+// A batch that the device's LDS holds at once with the roomiest visited table
+// has that one; visited_buckets is for larger ones.  (d 400, degree 16, beam 777
+// on a small set, 1,000 queries, four waves each: 1.70 ms at 99% load, 1.18 at 90%.)
+inline SearchParams launch_params(const SearchParams &P, int nw) {
+    const uint32_t b = visited_buckets_roomy(static_cast<uint32_t>(P.beam), static_cast<uint32_t>(P.degree));
+    if (b <= static_cast<uint32_t>(P.buckets)) return P;
+    SearchParams Q = P;
+    Q.buckets = static_cast<int>(b);
+    Q.lds = lds_layout(static_cast<uint32_t>(P.dim), static_cast<uint32_t>(P.padded_dim),
+                       static_cast<uint32_t>(P.pbeam), b);
+    const uint32_t bytes = nw > 1 ? Q.lds.total_team : Q.lds.total;
+    int dev = 0, cus = 0;
+    if (bytes > 65536u || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return P;
+    return P.nq <= static_cast<long long>(cus) * lds_groups(bytes) ? Q : P;
+}
+
 template <int WT, int DPL, int DIM_T, int DEG_T, bool BIG, int NW>
-void launch_form(const SearchParams &P, hipStream_t stream, bool count, bool prof) {
+void launch_form(const SearchParams &P0, hipStream_t stream, bool count, bool prof) {
+    const SearchParams P = launch_params(P0, NW);
     const dim3 grid(P.nq), block(64 * NW);
     const uint32_t lds = NW > 1 ? P.lds.total_team : P.lds.total;
     if (prof)

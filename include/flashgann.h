@@ -64,7 +64,7 @@ typedef struct {
     double elapsed_s;        /* host wall clock around launch + sync
                                 (gpu_search_adaptive.cu:98-107) */
     float kernel_ms;         /* HIP-event time of the search kernel */
-    uint32_t lds_bytes;      /* dynamic LDS per workgroup (one query) */
+    uint32_t lds_bytes;      /* dynamic LDS per workgroup (one query), as fg_lds_bytes */
     uint32_t visited_slots;  /* visited-table slots used by the kernel */
 } fg_stats;
 
@@ -162,7 +162,9 @@ int fg_search_profile(fg_index *index, const float *d_queries, uint32_t nq, uint
                       uint32_t *d_results, unsigned long long *d_phase, void *stream);
 
 /* Dynamic LDS bytes one query's workgroup needs (the analogue of
- * calculate_shared_mem_size, src/adaptive_search_utils.cuh:152-176). */
+ * calculate_shared_mem_size, src/adaptive_search_utils.cuh:152-176) in a launch
+ * larger than the device holds at once; a smaller one may have a roomier
+ * visited table. */
 uint32_t fg_lds_bytes(uint32_t dim, uint32_t beam, uint32_t degree);
 
 /* Waves per query (1, 2 or 4) that a search of nq queries at this K and beam
