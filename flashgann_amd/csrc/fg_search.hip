@@ -845,7 +845,7 @@ int launch_t(const SearchParams &P, hipStream_t stream, int *waves_only = nullpt
 
 // Whether a search may run as two launches (first slice, order, second
 // slice): searches that reach the suspension point, with suspended state of
-// at most kSliceMaxBytes (about 400,000 queries at d 128, beam 256).
+// at most kSliceMaxBytes (422,000 queries at d 128, beam 256).
 // slice_fits then asks for the one-wave form and a batch larger than the
 // device holds at once (the last queries to start are the ones that make a
 // launch's tail).  FLASHGANN_SLICE=0 / 1 forces one launch / two launches
@@ -872,9 +872,15 @@ uint64_t slice_buffer_words(const SearchParams &P, uint64_t *states_out, uint64_
 // fg_search_stream's largest launch of several batches.
 constexpr uint32_t kStreamQueries = 16384;
 
+// The limit counts 8 words of prepared query per code word (its levels and wrap
+// words in bits) where the digit rows take 13 and a row of zeros: which batches
+// run as two launches does not hang on how the levels are laid out.  The buffer
+// is at most half as large again as the limit (short beams, long vectors).
 bool slice_wanted(const SearchParams &P) {
     if (P.nq < 1 || P.max_iter <= kSliceStop) return false;
-    return slice_buffer_words(P, nullptr, nullptr) * 4u <= kSliceMaxBytes;
+    const uint32_t W = static_cast<uint32_t>(P.padded_dim) / 32u;
+    const uint64_t rows = static_cast<uint64_t>(P.nq) * (prep_words(W) - 8u * W);
+    return (slice_buffer_words(P, nullptr, nullptr) - rows) * 4u <= kSliceMaxBytes;
 }
 
 // slice_wanted's answer for a batch whose form is known: the one-wave form,

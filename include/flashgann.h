@@ -184,7 +184,8 @@ int fg_search_waves(fg_index *index, uint32_t nq, uint32_t K, uint32_t beam);
  * search of nq queries at this K and beam.  Two when the batch, in the
  * one-wave form, holds more queries than the device runs at once (6,144 at
  * d 128, degree 32, beam 256), for either metric, while the suspended state
- * stays within 1 GiB (about 400,000 queries at d 128, beam 256): every query
+ * stays within 1 GiB, of the prepared query 8 words per 32 dimensions counted
+ * (422,000 queries at d 128, beam 256): every query
  * first runs to iteration 15 and an unfinished one keeps its state (beam,
  * candidates, controller, counters and prepared query) in memory the index
  * holds, then the unfinished queries resume in a second launch, those with

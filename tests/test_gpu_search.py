@@ -526,6 +526,22 @@ def test_search_launches_reports_the_schedule(gpu_available, monkeypatch):
     ix.close()
 
 
+@pytest.mark.parametrize("dim,beam,most", [(128, 256, 422000), (1536, 640, 142000), (1100, 64, 366500),
+                                           (64, 1024, 124000)])
+def test_two_launch_limit(gpu_available, monkeypatch, dim, beam, most):
+    """The largest batch that runs as two launches, 1 GiB of suspended state at
+    20 + 2 (beam + 32) + 4 + 8 padded_dim / 32 words a query and three more for
+    the order, to within 1%, whatever words the prepared query takes."""
+    from flashgann_amd import Index
+    cb, _, _ = small_index(n=300, nq=4, dim=dim, comps=4)
+    ix = Index.from_codebook(cb)
+    monkeypatch.setenv("FLASHGANN_TEAM", "0")
+    monkeypatch.delenv("FLASHGANN_SLICE", raising=False)
+    assert ix.search_launches(most, 10, beam) == 2
+    assert ix.search_launches(most * 101 // 100, 10, beam) == 1
+    ix.close()
+
+
 @pytest.mark.parametrize("nq,beam", [(4000, 256), (4000, 384), (16384, 256), (16384, 512), (16385, 256),
                                      (30000, 384)])
 def test_two_launch_search_large_batches(gpu_available, monkeypatch, nq, beam):
