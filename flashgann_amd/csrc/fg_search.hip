@@ -911,6 +911,10 @@ int launch(fg_index *ix, const SearchParams &P0, hipStream_t stream, bool may_sl
             // area).  If it cannot be allocated, the search makes one launch.
             uint64_t states = 0, pad = 0;
             const uint64_t words = slice_buffer_words(P0, &states, &pad);
+            // (a buffer that has to grow may still be in use by a sliced search on
+            // another stream: that one ends before it is freed)
+            if (ix->slice_pending && words * 4u > ix->slice_cap)
+                FG_HIP(hipEventSynchronize(ix->slice_done), "wait for the last two-launch search");
             if (ensure(reinterpret_cast<void **>(&ix->d_slice), &ix->slice_cap, words * 4u) != FG_OK) {
                 (void)hipGetLastError();
                 return launch_t<false>(P0, stream, nullptr, true);

@@ -302,6 +302,39 @@ def test_search_stream_matches_single_launch(gpu_available, batch, nstreams):
     assert np.array_equal(got.numpy().view(np.uint32), oids)
 
 
+def test_two_launch_buffer_grows_behind_a_search(gpu_available, monkeypatch):
+    """A larger two-launch search on one stream, by either entry point, while a
+    smaller one on another has not ended: the state buffer that the first uses
+    is kept until then."""
+    import torch
+    from flashgann_amd import Index
+    from oracle import oracle as O
+    monkeypatch.setenv("FLASHGANN_TEAM", "0")
+    monkeypatch.setenv("FLASHGANN_SLICE", "1")
+    cb, q, _ = small_index(n=3000, nq=300)
+    rids, _ = O.OracleIndex.from_codebook(cb).search(q, 10, 128)
+    ix = Index.from_codebook(cb)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    sizes, dq, out = (300, 4000, 16000), [], []
+    for n in sizes:
+        dq.append(torch.as_tensor(q, device="cuda").repeat(-(-n // q.shape[0]), 1)[:n].contiguous())
+        out.append(torch.full((n, 10), -1, dtype=torch.int32, device="cuda"))
+    work = torch.ones((4096, 4096), device="cuda")
+    torch.cuda.synchronize()
+    for i, n in enumerate(sizes):
+        with torch.cuda.stream(streams[i]):
+            for _ in range(4):
+                work @ work
+        if i < 2:
+            ix.search_device(dq[i].data_ptr(), n, 10, 128, out[i].data_ptr(), 0, streams[i].cuda_stream)
+        else:
+            ix.search_stream(dq[i].data_ptr(), n, 10, 128, out[i].data_ptr(), 1000, 2, streams[i].cuda_stream)
+    torch.cuda.synchronize()
+    ix.close()
+    for n, o in zip(sizes, out):
+        assert np.array_equal(o.cpu().numpy().view(np.uint32), rids[np.arange(n) % q.shape[0]])
+
+
 @pytest.mark.parametrize("nq,batch,nstreams", [(16001, 1000, 2), (40000, 1000, 2), (40001, 9000, 4), (33000, 1, 1),
                                                (40000, 20000, 2), (50001, 16384, 8), (20000, 16383, 3)])
 def test_search_stream_several_launches(gpu_available, nq, batch, nstreams):
