@@ -4,7 +4,6 @@
 // kernels and launch function in its own object, so the classes compile in
 // parallel; fg_search.hip holds the host side and calls them.
 #pragma once
-// sees the visited set as of the round's start; the lowest (task, lane) wins".
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -99,12 +98,6 @@ __host__ __device__ inline int keep_limit(uint32_t active, int theta, float rho)
     return rho_keep < budget ? rho_keep : budget;
 }
 
-__host__ __device__ inline int keep_with_cutoff(int limit, bool kth_valid, uint32_t near) {
-    if (!kth_valid) return limit;
-    const int n = near < 1u ? 1 : static_cast<int>(near);
-    return n < limit ? n : limit;
-}
-
 // adaptive_search_utils.cuh:121-135
 __host__ __device__ inline int keep_count_for_expander(uint32_t active, int theta, float rho,
                                                        bool kth_valid, uint32_t near) {
@@ -185,7 +178,7 @@ __host__ __device__ __forceinline__ int list_spare(const uint32_t *list, const u
 }
 
 // The lead wave's way out of the search loop in the team form: it tells the
-// helper to stop at their meeting point (the helper then leaves too).
+// helpers to stop at their meeting point (they then leave too).
 template <int NW>
 __device__ __forceinline__ void team_stop(TeamBlock *tb, int lane) {
     if constexpr (NW > 1) {
@@ -414,30 +407,6 @@ __host__ __device__ constexpr uint64_t lane_bit_mask(int v) {
 // A uniform lane mask as this lane's bool (no instructions: the mask is the
 // condition register).
 __device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
-
-// Set bits in this lane's 32-lane half of a ballot: two scalar counts and
-// one select, instead of a per-lane 64-bit shift and count.
-__device__ __forceinline__ uint32_t half_popc(uint64_t m) {
-    const uint32_t lo = static_cast<uint32_t>(__popc(static_cast<uint32_t>(m)));
-    const uint32_t hi = static_cast<uint32_t>(__popc(static_cast<uint32_t>(m >> 32)));
-    return lane_in(0xFFFFFFFF00000000ull) ? hi : lo;
-}
-
-// Set bits in this lane's G-lane group of a ballot (G = 32: its half; G = 16:
-// its row), from scalar counts and selects.
-template <int G>
-__device__ __forceinline__ uint32_t group_popc(uint64_t m) {
-    if constexpr (G == 32) {
-        return half_popc(m);
-    } else {
-        const uint32_t r0 = static_cast<uint32_t>(__popc(static_cast<uint32_t>(m) & 0xFFFFu));
-        const uint32_t r1 = static_cast<uint32_t>(__popc(static_cast<uint32_t>(m) >> 16));
-        const uint32_t r2 = static_cast<uint32_t>(__popc(static_cast<uint32_t>(m >> 32) & 0xFFFFu));
-        const uint32_t r3 = static_cast<uint32_t>(__popc(static_cast<uint32_t>(m >> 48)));
-        const bool odd = lane_in(0xFFFF0000FFFF0000ull), high = lane_in(0xFFFFFFFF00000000ull);
-        return high ? (odd ? r3 : r2) : (odd ? r1 : r0);
-    }
-}
 
 // Lane i reads lane i ^ m, all lanes active.  m < 16 stays inside a 16-lane
 // row: DPP quad_perm (1, 2), half-row mirror then quad reverse
@@ -1926,8 +1895,8 @@ __device__ __forceinline__ void hash_contains_n(const uint32_t *t, uint32_t nb, 
 // dimension 256 gets 4, and the wide runtime geometry 3 (<= 168 VGPRs) for its
 // code batches: at padded dimension 2048 its LDS holds it to about 3 anyway.
 // NW = 2 or 4: the team form (two or four waves per query; see TeamBlock).  Wave 0 leads:
-// it runs every phase, the helper wave joins it in stage II's rounds and the
-// exact distances; `lead_sync` orders the lead wave's own LDS accesses and
+// it runs every phase; the helpers join it in stage II's rounds, the exact
+// distances, the visited-table rebuild and, at beams over 256, the merge; `lead_sync` orders the lead wave's own LDS accesses and
 // the workgroup barriers mark the meeting points.
 template <int WT, int DPL, int DIM_T, int DEG_T, bool COUNT, bool PROF, bool BIG, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0 ? (NW == 4 ? 4 : 3) : WT > 4 ? 4 : (NW == 1 && !COUNT && !PROF && (!BIG || WT == 2) && (DIM_T > 0 || DPL < 4) ? 6 : 5)))) void fg_search_kernel(SearchParams P) {
@@ -2058,7 +2027,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
         lead_sync<NW>();
     }
     if constexpr (NW > 1) {
-        // the quantised query's constants, for the helper
+        // the quantised query's constants, for the helpers
         if (lead && lane == 0) {
             tb->sum_q = static_cast<uint32_t>(sum_q);
             tb->qwidth_bits = __float_as_uint(qwidth);
@@ -2152,13 +2121,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
         // lane-derived values are recomputed in each iteration, not held
         const int lane = lane_id_opaque();
         const int h = lane >> 5, nl = lane & 31;
-        // the iteration's uniform state; the lead wave computes it, a helper
-        // wave receives it at the meeting point below
+        // the iteration's uniform state; the lead wave computes it, the
+        // helpers receive it at the meeting point below
         float kth = FLT_MAX, rho = 0.0f;
         int theta = 1;
         uint32_t nexp = 0;
         if (((iter + 1) % kHashReset) == 0) {  // adaptive_search.cuh:128-134
-            // (a team's waves take half each; the second meeting is before the
+            // (a team's waves take equal shares; the second meeting is before the
             // merge, which rewrites the beam they read)
             const int tid = NW > 1 ? lane + 64 * wv : lane;
             hash_reset(H, nbk, tid, 64 * NW);
@@ -2351,10 +2320,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                     // dispatch_candidate_bitonic_sort over the cbs-entry buffer (padding beyond it)
                     const float sk = nl < cbs ? dist : FLT_MAX;
                     const uint32_t sv = nl < cbs ? child : kMaxIndex;
-                    // (the runtime geometry of padded dimension 64 and 128 has no
-                    // registers left for the counted sort here as well, and in
-                    // the one-wave fixed-geometry kernels of degree 32 it would
-                    // cost a wave per SIMD)
+                    // (no counted sort here in the one-wave kernels of padded
+                    // dimension 64 and 128 but degree 16's: it would cost them a
+                    // wave per SIMD.  The team kernels of the runtime geometry
+                    // there hold 45 to 75 registers and could take it; not
+                    // measured)
                     const bool clean = ((kFixedGeo && (NW > 1 || DEG_T == 16)) || WT == 0 || WT > 4) &&
                                        !any_lane(!(((sk > -FLT_MAX) & (sk < FLT_MAX) & (sv != kMaxIndex)) |
                                                    ((sk == FLT_MAX) & (sv == kMaxIndex))));
@@ -2418,7 +2388,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
             for (int rbase = 0; rbase < tasks; rbase += kSearchWidth) {
                 constexpr int SR = kSearchWidth / TPW;  // sub-rounds of TPW tasks
                 // this wave's sub-rounds: all of them, or in the team form
-                // the first half (lead) or the second (helper)
+                // its equal share of them, the lead wave's first
                 constexpr int SRN = SR / NW;
                 const int sr0 = wv * SRN;
                 uint32_t cid[SRN];
@@ -2601,8 +2571,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                         // near, and the near smallest (value, lane) pairs are the
                         // ones at or below the cutoff: every such lane ranks
                         // ahead of every lane above it.  No selection rounds.
-                        // Otherwise keep_with_cutoff's count: one for near = 0
-                        // with a valid cutoff, else the limit.
+                        // Otherwise one for near = 0 with a valid cutoff, else
+                        // the limit (keep_limit).
                         int k = near > lim[sr][t] ? lim[sr][t] : 0;
                         k = near == 0 ? (kth_valid ? 1 : lim[sr][t]) : k;
                         k &= static_cast<int>(nd);
@@ -2688,7 +2658,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WT == 0
                     lead_sync<NW>();
                 }
                 // in the team form the round's inserts are in the table before
-                // the helper's visited tests of the next round
+                // the helpers' visited tests of the next round
                 if constexpr (NW > 1) {
                     if (rbase + kSearchWidth < tasks) __syncthreads();
                 }

@@ -6,9 +6,9 @@
 //   * one workgroup = one wave = one query; the reference's 256-thread block
 //     barriers become wave-ordered LDS traffic, so the beam, candidate buffer,
 //     visited table and controller state never leave the CU's LDS/registers
-//     (where a second wave costs no query a slot the team form runs instead: a
-//     second wave per query takes half of the expansion rounds and of the
-//     exact distances);
+//     (where further waves cost no query a slot a team form runs instead: two
+//     or four waves per query share the expansion rounds, the exact distances
+//     and, at beams over 256, the merge);
 //   * the reference's 32-lane sorting networks are data-oblivious, so the
 //     same compare-exchange sequence is replayed on the wave (two 32-lane
 //     halves, or 1-2 positions per lane) and ties resolve identically;
@@ -353,8 +353,13 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 // passes over padded_dim doubles per edge; the fast transform in registers
 // leaves one read of each neighbour's vector and one write of the row, and
 // the row leaves the device whole: 50k points at d 128, degree 32 into a host
-// codebook 27.1 -> 2.9 ms (77 MB of rows through page-locked staging; the
-// copy, not this kernel, bounds it).  padded_dim = 64 K.
+// codebook 27.1 -> 2.9 ms (77 MB of rows through page-locked staging).  There
+// the copies bound it: an 8 MB block takes this kernel 108 us, the copy to the
+// host 147 and the one into the result some 300.  Longer vectors are bound by
+// the kernel, whose registers leave few waves (three a SIMD at K = 16, one at
+// 32) and whose blocks hold few rows: 250 us a block at d 960, 438 at d 1536,
+// 505 at d 2048.  8k points of degree 32: d 960 36.9 -> 4.1 ms, d 1536 137 ->
+// 9.6; 5k at d 2048 109 -> 7.7.  padded_dim = 64 K.
 template <int K>
 __global__ __launch_bounds__(64) void fg_encode_kernel(EncodeParams E) {
     __shared__ double pc[64 * K];  // the rotated vector of the node
@@ -1178,8 +1183,9 @@ int fg_search_stream(fg_index *ix, const float *d_queries, uint32_t nq, uint32_t
     // small batch leaves most of the device idle and ends in a tail of its
     // longest searches, and one launch of them all pays both once.  8 batches
     // of 1,000 queries (d 128, beam 128) on two streams: 1.002 -> 0.515 ms.
-    // The bound keeps a launch's two-launch state small (40 MB at beam 256)
-    // and its order step in one workgroup.
+    // The bound keeps what a call holds small (two-launch state of 40 MB at beam
+    // 256); it is not where larger launches stop paying: 80,000 queries at beam
+    // 256 in 8 launches on two streams 8.78 M queries/s, in one 10.35 M.
     const uint32_t per = batch < kStreamQueries ? batch * (kStreamQueries / batch) : batch;
     if (nq <= per) {
         P.nq = static_cast<int>(nq);
@@ -1279,8 +1285,10 @@ int search_host(fg_index *ix, SearchParams &P, const float *queries, uint32_t nq
 }
 
 // A small host-buffer search: the kernel reads the queries from page-locked
-// host memory (once per query: padded dimensions up to 256 keep a query in
-// registers) and writes the ids there, so the call makes no copy of its own.
+// host memory and writes the ids there, so the call makes no copy of its own.
+// (A query is read a few times over: by its preparation, by each wave into
+// registers, which padded dimensions up to 256 hold, and for the entry point's
+// distance; a query resumed by the second slice, into registers again.)
 // Each copy is a blocking call of some 15 us for any size: one query at d 128,
 // beam 64 took 156 us with them and takes 122, 256 queries at K 100 403 and 352.
 // The line at kHostStage is where copying through the

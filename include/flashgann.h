@@ -143,7 +143,10 @@ int fg_search_device(fg_index *index, const float *d_queries, uint32_t nq, uint3
  * `stream`, as fg_search_device would.  Results land in query order in
  * d_results (nq x K); each query's ids are those fg_search_device returns.
  * All batches run after the work already queued on `stream` and that stream's
- * later work waits for all of them; the call returns without synchronising.
+ * later work waits for all of them; the call returns without synchronising
+ * (but see fg_search_launches: a call of one launch that runs as two allocates
+ * the index's state buffer on first use and when a larger batch needs more,
+ * which synchronises the device).
  * Calls on one index share its internal streams: issue them from one host
  * thread. */
 int fg_search_stream(fg_index *index, const float *d_queries, uint32_t nq, uint32_t K, uint32_t beam,

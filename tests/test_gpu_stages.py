@@ -86,9 +86,9 @@ def _wrap_queries(signs, B, count, seed=12):
 
 @pytest.mark.parametrize("dim", [64, 256, 512, 1024, 2048])
 def test_wrap_chunks_scores_and_search(gpu_available, dim):
-    """The popcount planes' wrap correction reproduces the uint8 LUT, for
-    each code width the estimators have: 2 words (fixed geometry) and 8, 16,
-    32 and 2 x 32 words (generic geometry)."""
+    """The wrap words' correction reproduces the uint8 LUT, for each code width
+    the estimators have: 2 and 8 words in registers, 16, 32 and 2 x 32 words
+    read in spans."""
     from flashgann_amd import Index
     from oracle import oracle as O
     cb, _, _ = small_index(n=1200, nq=4, dim=dim, comps=8)
